@@ -58,8 +58,12 @@ template <uint32_t K> __global__ void k_gemm_down(const _Float16*, ExpertTiles, 
 __global__ void k_gemm_dense(const _Float16*, uint32_t, DenseSegs, float*, uint32_t, size_t);
 __global__ void k_pf_embed(DevMat, const uint32_t*, uint32_t, uint32_t, float*, DevState*);
 __global__ void k_tile_gemm(DevMat, uint32_t, uint8_t*);
+template <int MB>
+__global__ void k_gemm_dense_skinny(const _Float16*, uint32_t, DenseSegs, float*, uint32_t, size_t);
+template <int Z>
 __global__ void k_pf_norm(float*, const float*, uint32_t, float, _Float16*, float*, const float*, size_t, uint32_t*);
-__global__ void k_pf_qkrope(const float*, const float*, const float*, const float2*, uint32_t, uint32_t, uint32_t,
+template <int Z>
+__global__ void k_pf_qkrope(const float*, size_t, const float*, const float*, const float2*, uint32_t, uint32_t, uint32_t,
                             uint32_t, uint32_t, float, _Float16*, float*, float*, _Float16*, _Float16*, uint32_t,
                             uint32_t*);
 __global__ void k_pf_attn(const _Float16*, const _Float16*, const _Float16*, uint32_t, uint32_t, uint32_t, uint32_t,
@@ -988,13 +992,16 @@ void prefill_alloc(qh_ctx* c, uint32_t cap) {
     const uint32_t max_tiles = (uint32_t)((n_asg + 127) / 128 + d.experts);
     auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
     const uint64_t npair = ((cap + 15) / 16 + 1) / 2 * d.kvheads;  // attention block pairs
+    // a dense launch with more than one column split writes at most
+    // kPfDenseUnits 128 x 128 tiles (pf_dense)
+    const uint64_t split_floats = kPfDenseUnits * 128ull * 128ull;
     struct R {
         uint64_t bytes;
         void** dst;
     } regs[] = {
         {cap * H * 4, (void**)&P.X},           {cap * H * 4, (void**)&P.Xn32},
-        {cap * (qd + 2 * kvd) * 4, (void**)&P.QKV}, {(uint64_t)cap * d.experts * 4 * kPfRouterSplit, (void**)&P.LR},
-        {n_asg * 4, (void**)&P.wts},           {std::max<uint64_t>(n_asg, 2ull * cap) * H * 4, (void**)&P.Y},
+        {std::max<uint64_t>(cap * (qd + 2 * kvd), split_floats) * 4, (void**)&P.QKV}, {(uint64_t)cap * d.experts * 4 * kPfRouterSplit, (void**)&P.LR},
+        {n_asg * 4, (void**)&P.wts},           {std::max<uint64_t>(n_asg * H, split_floats) * 4, (void**)&P.Y},
         {cap * H * 2, (void**)&P.Xn16},        {(uint64_t)d.heads * cap * 128 * 2, (void**)&P.Q16},
         {cap * qd * 2, (void**)&P.O16},        {n_asg * d.ff * 2, (void**)&P.Hs},
         {n_asg * 4, (void**)&P.ids},           {(uint64_t)(d.experts + 1) * 4, (void**)&P.goff},
@@ -1030,17 +1037,20 @@ template <class F> void dispatch_km(uint32_t kind, F f) {
 }
 
 // C[t][cofs_i + n] = X16[t] . W_i[n] for t < S and each matrix i of `mats`
-// (one launch; with `splits` > 1 the columns are split in equal parts, part z
-// written to C + z * split_stride): the MFMA GEMM on the quantised rows
-// (dequantised into the tiles).
-void pf_dense(qh_ctx* c, std::initializer_list<std::pair<const DevMat*, uint32_t>> mats, const _Float16* X16,
-              uint32_t S, float* C, uint32_t ldc, uint32_t splits = 1, size_t split_stride = 0) {
+// (one launch; the columns are split in the returned number of equal parts,
+// part z written to C + z * S * ldc): the MFMA GEMM on the quantised rows
+// (dequantised into the tiles).  The split keeps the chip full when the tiles
+// alone would not: doubled while the workgroups fit kPfDenseUnits (one round
+// of three per CU) and a part is whole 256-column super-blocks.
+uint32_t pf_dense(qh_ctx* c, std::initializer_list<std::pair<const DevMat*, uint32_t>> mats, const _Float16* X16,
+                  uint32_t S, float* C, uint32_t ldc) {
     DenseSegs G{};
-    uint32_t tiles = 0;
+    uint32_t tiles = 0, cols = 0;
     for (const auto& m : mats) {
         const DevMat& W = *m.first;
         if (!block_kind(W.kind)) throw Error("prefill projection is not block-quantised");
-        if ((W.cols / splits) % 256 || W.cols % splits) throw Error("prefill projection width does not split");
+        if (W.cols % 256 || (cols && W.cols != cols)) throw Error("prefill projection width does not split");
+        cols = W.cols;
         G.W[G.n] = W;
         tiles += (W.rows + 127) / 128;
         G.tile_end[G.n] = tiles;
@@ -1048,8 +1058,28 @@ void pf_dense(qh_ctx* c, std::initializer_list<std::pair<const DevMat*, uint32_t
         G.n++;
     }
     for (uint32_t i = G.n; i < 3; i++) G.tile_end[i] = tiles;
-    hipLaunchKernelGGL(k_gemm_dense, dim3(8 * ((S + 1023) / 1024) * tiles, 1, splits), dim3(256), 0, c->s, X16, S, G, C, ldc,
-                       split_stride);
+    const uint32_t units = (S + 127) / 128 * tiles;
+    uint32_t splits = 1;
+    while (splits < 8 && (cols / 256) % (2 * splits) == 0 && units * 2 * splits <= kPfDenseUnits) splits *= 2;
+    const size_t stride = (size_t)S * ldc;
+    if (S <= kPfSkinny / 2)
+        hipLaunchKernelGGL(k_gemm_dense_skinny<1>, dim3(tiles, 1, splits), dim3(256), 0, c->s, X16, S, G, C, ldc, stride);
+    else if (S <= kPfSkinny)
+        hipLaunchKernelGGL(k_gemm_dense_skinny<2>, dim3(tiles, 1, splits), dim3(256), 0, c->s, X16, S, G, C, ldc, stride);
+    else
+        hipLaunchKernelGGL(k_gemm_dense, dim3(8 * ((units + 7) / 8), 1, splits), dim3(256), 0, c->s, X16, S, G, C, ldc,
+                           stride);
+    return splits;
+}
+
+// Calls f with the split count as a compile-time constant.
+template <class F> void dispatch_splits(uint32_t z, F f) {
+    switch (z) {
+    case 1: f(std::integral_constant<int, 1>{}); break;
+    case 2: f(std::integral_constant<int, 2>{}); break;
+    case 4: f(std::integral_constant<int, 4>{}); break;
+    default: f(std::integral_constant<int, 8>{}); break;
+    }
 }
 
 // One decoder layer (src/model.rs:227-287) for chunk tokens [0, S) at
@@ -1061,26 +1091,34 @@ void prefill_layer(qh_ctx* c, size_t l, uint32_t S, uint32_t p0) {
     const uint32_t H = d.hidden, qd = d.heads * 128, kvd = d.kvheads * 128, row = qd + 2 * kvd;
     uint32_t* err = &c->acts.st->err;  // kErrRange: an fp16 operand out of range
     if (l == 0)  // later layers: written by the previous layer's combine
-        hipLaunchKernelGGL(k_pf_norm, dim3(S), dim3(kBlock), 0, c->s, P.X, L.attn_norm, H, d.eps, P.Xn16,
+        hipLaunchKernelGGL(k_pf_norm<0>, dim3(S), dim3(kBlock), 0, c->s, P.X, L.attn_norm, H, d.eps, P.Xn16,
                            (float*)nullptr, (const float*)nullptr, (size_t)0, err);
     // q | k | v: one launch over the three quantised matrices, QKV[t] = [q | k | v]
-    pf_dense(c, {{&L.q, 0u}, {&L.k, qd}, {&L.v, qd + kvd}}, P.Xn16, S, P.QKV, row);
+    const uint32_t zq = pf_dense(c, {{&L.q, 0u}, {&L.k, qd}, {&L.v, qd + kvd}}, P.Xn16, S, P.QKV, row);
     const uint32_t vp = (d.ctx + 63) / 64 * 64;  // row pitch of the transposed V copy
     if (p0 > 0)  // fp16 copies of this layer's earlier positions
         hipLaunchKernelGGL(k_pf_kvh, dim3(p0), dim3(kBlock), 0, c->s, L.kcache, L.vcache, 0u, d.kvheads, d.ctx, vp,
                            P.Kh, P.Vth);
-    hipLaunchKernelGGL(k_pf_qkrope, dim3(S), dim3(kBlock), 0, c->s, P.QKV, L.q_norm, L.k_norm, c->acts.rope, p0, S,
-                       d.heads, d.kvheads, d.ctx, d.eps, P.Q16, L.kcache, L.vcache, P.Kh, P.Vth, vp, err);
+    // with split sums (a short prompt) a token's head slots are spread over
+    // several workgroups, one round of loads per wave
+    dispatch_splits(zq, [&](auto Z) {
+        constexpr int z = decltype(Z)::value;
+        const uint32_t per = kWaves * qkrope_slots(z), wgs = z == 1 ? 1 : (d.heads + 2 * d.kvheads + per - 1) / per;
+        hipLaunchKernelGGL(k_pf_qkrope<z>, dim3(S, wgs), dim3(kBlock), 0, c->s, P.QKV, (size_t)S * row, L.q_norm,
+                           L.k_norm, c->acts.rope, p0, S, d.heads, d.kvheads, d.ctx, d.eps, P.Q16, L.kcache, L.vcache,
+                           P.Kh, P.Vth, vp, err);
+    });
     // two workgroups per pair of query blocks (the n-1-i-th and the i-th of n)
     const uint32_t npair = ((S + 15) / 16 + 1) / 2;
     hipLaunchKernelGGL(k_pf_attn, dim3(2 * npair * d.kvheads), dim3(256), 0, c->s, P.Q16, P.Kh, P.Vth, p0, S,
                        d.heads / d.kvheads, d.ctx, vp, qd, P.O16, P.axw, P.axc);
-    // o in two column halves (twice the workgroups) into Y's space; the norm
-    // adds both to the residual (model.rs:246-248) before normalising
-    const size_t ostride = (size_t)S * H;
-    pf_dense(c, {{&L.o, 0u}}, P.O16, S, P.Y, H, 2, ostride);
-    hipLaunchKernelGGL(k_pf_norm, dim3(S), dim3(kBlock), 0, c->s, P.X, L.ffn_norm, H, d.eps, P.Xn16, P.Xn32,
-                       (const float*)P.Y, ostride, err);
+    // o's column splits go to Y's space; the norm adds them to the residual
+    // (model.rs:246-248) before normalising
+    const uint32_t zo = pf_dense(c, {{&L.o, 0u}}, P.O16, S, P.Y, H);
+    dispatch_splits(zo, [&](auto Z) {
+        hipLaunchKernelGGL(k_pf_norm<decltype(Z)::value>, dim3(S), dim3(kBlock), 0, c->s, P.X, L.ffn_norm, H, d.eps,
+                           P.Xn16, P.Xn32, (const float*)P.Y, (size_t)S * H, err);
+    });
     hipLaunchKernelGGL(k_pf_router, dim3((S + 63) / 64, kPfRouterSplit), dim3(kBlock), 0, c->s, P.Xn32, L.router,
                        S, H, d.experts, P.LR);
     hipLaunchKernelGGL(k_pf_topk, dim3((S + kWaves - 1) / kWaves), dim3(kBlock), 0, c->s, P.LR, S,

@@ -207,6 +207,15 @@ void launch_sample_fold(const SampleArgs& a, const unsigned long long* cand, flo
 // order).
 constexpr uint32_t kPfRouterSplit = 8;
 
+// Column splits of the batched prefill's dense projections: 1, 2, 4 or 8
+// partial sums, added in split order by the kernel that reads them.  Row tiles
+// x column tiles of a launch, times its splits, stay within
+// kPfDenseUnits workgroups (three per CU).
+constexpr uint32_t kPfDenseUnits = 768;
+constexpr uint32_t kPfSkinny = 64;  // most tokens of the skinny dense kernel (prefill.hip: k_gemm_dense_skinny)
+// Head slots per wave and round of k_pf_qkrope<Z>.
+QH_HD constexpr uint32_t qkrope_slots(uint32_t z) { return z == 1 ? 5 : z == 2 ? 2 : 1; }
+
 // Batched-prefill attention (prefill.hip: k_pf_attn): floats of the (O, m, l)
 // hand-over slot of one workgroup (4 waves x 68 values x 64 lanes) when two
 // workgroups share a query block's keys; two slots and a zeroed counter per

@@ -372,6 +372,89 @@ __device__ __forceinline__ void gemm_tile_r(const _Float16* const (&arows)[4], c
     }
 }
 
+// The same product for a tile of at most 32 MB rows (MB = 1, 2): a prompt or
+// an expert with few rows.  There the weights' bytes bound the launch, not the
+// products, so the loop is built to keep more of them in flight: a step is one
+// whole 256-column super-block (32 or 64 KB of weights per workgroup requested
+// one step ahead, each row's header once instead of once per slice), the
+// activations of 256 / MB columns are staged per barrier, and the unused row
+// blocks cost no registers.  acc[nb][mb] += A[m0 .. m0 + 32 MB) x
+// W_nb[n0 .. n0+128)^T over super-blocks [sb0, sb0 + nsb); arows[i]: the A row
+// of tile row srow_row<MB>(i) (any valid row past the tile's rows).
+constexpr int kSP(int mb) { return 256 / mb + 8; }                 // LDS row pitch in halfs
+constexpr int kRS = 2 * 32 * (256 + 8);                            // halfs of LDS, MB = 1
+constexpr int kRS2 = 2 * 64 * (128 + 8);                           // halfs of LDS, MB = 2
+template <int MB> __device__ __forceinline__ uint32_t srow_row(uint32_t i) {
+    return (threadIdx.x + kGT * i) / (32 / MB);  // 32 / MB 16-byte chunks per staged row
+}
+template <uint32_t KIND, int NB, int MB>
+__device__ __forceinline__ void gemm_skinny(const _Float16* const (&arows)[4], const uint8_t* const (&wblk)[NB],
+                                            uint32_t sb0, uint32_t nsb, f16v (&acc)[NB][MB], _Float16* As) {
+    constexpr int KS = 4 / MB, P = kSP(MB);  // slices per staged part, LDS pitch
+    const uint32_t lane = threadIdx.x & 63, grp = lane >> 5;
+    const uint32_t ach = threadIdx.x % (32 / MB);
+    WReg<KIND> wr[2][NB][4];
+    uint4 av[4];
+    auto wload = [&](auto B_, uint32_t i) {
+        const size_t o = (size_t)(sb0 + min(i, nsb - 1)) * tile_block_bytes(KIND);  // past the end: a harmless reload
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int sl = 0; sl < 4; sl++) wr[decltype(B_)::value][nb][sl].load(wblk[nb] + o, sl, lane);
+    };
+    auto aload = [&](uint32_t j) {  // staged part j: columns 256 sb0 + 64 KS j ..
+        const uint32_t k0 = 256 * sb0 + 64 * KS * min(j, MB * nsb - 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) av[i] = gld<uint4>(arows[i] + k0 + 8 * ach);
+    };
+    aload(0);
+    wload(std::integral_constant<int, 0>{}, 0);
+    auto step = [&](auto B_, uint32_t i) {
+        constexpr int B = decltype(B_)::value;
+#pragma unroll
+        for (int part = 0; part < MB; part++) {
+            const uint32_t j = MB * i + part;
+            _Float16* Ab = As + (j & 1) * 32 * MB * P;
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                *reinterpret_cast<uint4*>(Ab + srow_row<MB>(r) * P + 8 * ach) = av[r];
+            aload(j + 1);
+            if (part == 0) wload(std::integral_constant<int, 1 - B>{}, i + 1);
+            __syncthreads();  // the buffer's readers of part j - 2 passed the barrier of part j - 1
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) {
+                const int sl = KS * part + ks;
+                typename WReg<KIND>::Sc sc[NB];
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++) sc[nb] = wr[B][nb][sl].prep(sl, grp);
+                auto kstep = [&](auto S_) {
+                    constexpr int S = decltype(S_)::value;
+                    const uint32_t col = 64 * ks + 32 * (S >> 1) + 16 * grp + 8 * (S & 1);
+                    h8v af[MB];
+#pragma unroll
+                    for (int mb = 0; mb < MB; mb++)
+                        af[mb] = *reinterpret_cast<const h8v*>(Ab + (32 * mb + (lane & 31)) * P + col);
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++) {
+                        const h8v bf = wr[B][nb][sl].template dequant<S>(sc[nb], sl & 1);
+#pragma unroll
+                        for (int mb = 0; mb < MB; mb++)
+                            acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf, acc[nb][mb], 0, 0, 0);
+                    }
+                };
+                kstep(std::integral_constant<int, 0>{});
+                kstep(std::integral_constant<int, 1>{});
+                kstep(std::integral_constant<int, 2>{});
+                kstep(std::integral_constant<int, 3>{});
+            }
+        }
+    };
+    for (uint32_t i = 0; i < nsb; i += 2) {
+        step(std::integral_constant<int, 0>{}, i);
+        if (i + 1 < nsb) step(std::integral_constant<int, 1>{}, i + 1);  // workgroup-uniform
+    }
+}
+
 // XCD-aware tile order.  Workgroup b runs on XCD b % 8 (each XCD has its own
 // L2).  The grid is 1-D: XCD x takes the row tiles t = x, x + 8, ... and, for
 // each in turn, all nn column tiles, so that one row tile's activations (read
@@ -492,15 +575,26 @@ __device__ __forceinline__ void dense_body(const _Float16* X16, uint32_t S, cons
         }
 }
 
+// Unit u of the launch's `units`, so that every XCD (workgroup b runs on XCD
+// b % 8) takes one contiguous eighth of them, whatever their number: with the
+// row tiles dealt out in turn (xcd_tile), a prompt of at most 128 tokens ran
+// on one XCD and one of 384 on three (331 tokens with this and the column
+// splits: 30-40 -> 17-24 us per launch).  The grid holds 8 * ceil(units / 8)
+// workgroups; those past the end return units.
+__device__ __forceinline__ uint32_t xcd_unit(uint32_t units) {
+    const uint32_t per = (units + 7) / 8, u = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    return (blockIdx.x >> 3) < per ? min(u, units) : units;
+}
+
 // Three workgroups per CU (168 VGPRs, 4 of them spilled): the q|k|v grid of
 // 16 x 40 tiles at 2,048 tokens then runs in one round of 768 workgroup slots
 // rather than 1.25 rounds of 512.
 __global__ __launch_bounds__(kGT, 3) void k_gemm_dense(const _Float16* X16, uint32_t S, DenseSegs G, float* C,
                                                     uint32_t ldc, size_t split_stride) {
     __shared__ __align__(16) _Float16 smem[kRA];
-    uint32_t mt, t;
-    xcd_tile(G.tile_end[2], mt, t);  // row tile (tokens), column tile
-    if (mt * kGM >= S) return;
+    const uint32_t nt = G.tile_end[2], units = (S + kGM - 1) / kGM * nt, u = xcd_unit(units);
+    if (u >= units) return;
+    const uint32_t mt = u / nt, t = u % nt;  // row tile (tokens), column tile
     const uint32_t i = t < G.tile_end[0] ? 0 : t < G.tile_end[1] ? 1 : 2;  // workgroup-uniform
     const uint32_t t0 = i == 0 ? 0 : G.tile_end[i - 1];
     const DevMat& W = G.W[i];
@@ -514,6 +608,55 @@ __global__ __launch_bounds__(kGT, 3) void k_gemm_dense(const _Float16* X16, uint
     default: break;
     }
 }
+
+// k_gemm_dense for S <= 32 MB tokens (one row tile): gridDim.x column tiles x
+// gridDim.z column splits of whole super-blocks.  Bound by one round trip for
+// the weights (4.7-5.9 MB per launch): at 24 tokens a launch takes 5.4-6.4 us,
+// against 26-33 us in k_gemm_dense with 40 workgroups on one XCD.
+template <uint32_t KIND, int MB>
+__device__ __forceinline__ void dense_skinny_body(const _Float16* X16, uint32_t S, const DevMat& W, uint32_t n0,
+                                                  uint32_t sb0, uint32_t nsb, float* C, uint32_t ldc, uint32_t cofs,
+                                                  _Float16* smem) {
+    const uint32_t N = W.rows, ld = W.cols;
+    const _Float16* arows[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) arows[i] = X16 + (size_t)min(srow_row<MB>(i), S - 1) * ld;
+    const uint8_t* const wblk[1] = {
+        W.wt + (size_t)min((n0 >> 5) + (threadIdx.x >> 6), N / 32 - 1) * tile_group_bytes(KIND, W.cols)};
+    f16v acc[1][MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) acc[0][mb] = f16v{};
+    gemm_skinny<KIND, 1, MB>(arows, wblk, sb0, nsb, acc, smem);
+    const uint32_t n = n0 + racc_col();
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t m = racc_row(mb, i);
+            if (m < S && n < N) C[(size_t)m * ldc + cofs + n] = acc[0][mb][i];
+        }
+}
+
+template <int MB>
+__global__ __launch_bounds__(kGT, 2) void k_gemm_dense_skinny(const _Float16* X16, uint32_t S, DenseSegs G, float* C,
+                                                              uint32_t ldc, size_t split_stride) {
+    __shared__ __align__(16) _Float16 smem[MB == 1 ? kRS : kRS2];
+    const uint32_t t = blockIdx.x;
+    const uint32_t i = t < G.tile_end[0] ? 0 : t < G.tile_end[1] ? 1 : 2;  // workgroup-uniform
+    const uint32_t t0 = i == 0 ? 0 : G.tile_end[i - 1];
+    const DevMat& W = G.W[i];
+    const uint32_t nsb = W.cols / 256 / gridDim.z, sb0 = blockIdx.z * nsb;
+    float* Cz = C + blockIdx.z * split_stride;
+    switch (W.kind) {
+#define QH_DENSE(KD) \
+    case KD: dense_skinny_body<KD, MB>(X16, S, W, (t - t0) * kGN, sb0, nsb, Cz, ldc, G.cofs[i], smem); break;
+        QH_DENSE(Q4_0) QH_DENSE(Q8_0) QH_DENSE(Q4_K) QH_DENSE(Q5_K) QH_DENSE(Q6_K)
+#undef QH_DENSE
+    default: break;
+    }
+}
+template __global__ void k_gemm_dense_skinny<1>(const _Float16*, uint32_t, DenseSegs, float*, uint32_t, size_t);
+template __global__ void k_gemm_dense_skinny<2>(const _Float16*, uint32_t, DenseSegs, float*, uint32_t, size_t);
 
 // ------------------------------------------------------- tile layout --
 // Row-layout source byte of byte o of tile block (G, b) of a matrix whose
@@ -613,22 +756,25 @@ __global__ __launch_bounds__(kBlock) void k_pf_embed(DevMat emb, const uint32_t*
 }
 
 // RMSNorm (ops.rs:3-15) of row t: fp16 copy (GEMM input), optional fp32 copy.
-// With P: first X[t] += P[0][t] + P[1][t] (the two column halves of the
-// o-projection: the residual add of model.rs:246-248, in that order).
+// With Z > 0: first X[t] += P[0][t] + .. + P[Z-1][t] (the column splits of the
+// o-projection, added in split order: the residual add of model.rs:246-248).
+template <int Z>
 __global__ __launch_bounds__(kBlock) void k_pf_norm(float* X, const float* w, uint32_t H, float eps,
                                                     _Float16* Y16, float* Y32, const float* P, size_t pstride,
                                                     uint32_t* err) {
     __shared__ float red[kWaves];
     const size_t t = blockIdx.x;
     float* x = X + t * H;
-    if (P) {
-        const float* p0 = P + t * H;
-        const float* p1 = p0 + pstride;
+    if constexpr (Z > 0) {
+        const float* p = P + t * H;
         for (uint32_t i4 = threadIdx.x; 4 * i4 < H; i4 += kBlock) {
-            const float4 v = reinterpret_cast<const float4*>(x)[i4], a = reinterpret_cast<const float4*>(p0)[i4],
-                         b = reinterpret_cast<const float4*>(p1)[i4];
-            reinterpret_cast<float4*>(x)[i4] =
-                make_float4(v.x + (a.x + b.x), v.y + (a.y + b.y), v.z + (a.z + b.z), v.w + (a.w + b.w));
+            float4 v = reinterpret_cast<const float4*>(x)[i4], a[Z];
+#pragma unroll
+            for (int z = 0; z < Z; z++) a[z] = reinterpret_cast<const float4*>(p + z * pstride)[i4];
+#pragma unroll
+            for (int z = 1; z < Z; z++)
+                a[0] = make_float4(a[0].x + a[z].x, a[0].y + a[z].y, a[0].z + a[z].z, a[0].w + a[z].w);
+            reinterpret_cast<float4*>(x)[i4] = make_float4(v.x + a[0].x, v.y + a[0].y, v.z + a[0].z, v.w + a[0].w);
         }
         // each thread reads back only the elements it wrote
     }
@@ -658,36 +804,64 @@ __global__ __launch_bounds__(kBlock) void k_pf_norm(float* X, const float* w, ui
     note_range(bad, err);
 }
 
+template __global__ void k_pf_norm<0>(float*, const float*, uint32_t, float, _Float16*, float*, const float*, size_t,
+                                      uint32_t*);
+template __global__ void k_pf_norm<1>(float*, const float*, uint32_t, float, _Float16*, float*, const float*, size_t,
+                                      uint32_t*);
+template __global__ void k_pf_norm<2>(float*, const float*, uint32_t, float, _Float16*, float*, const float*, size_t,
+                                      uint32_t*);
+template __global__ void k_pf_norm<4>(float*, const float*, uint32_t, float, _Float16*, float*, const float*, size_t,
+                                      uint32_t*);
+template __global__ void k_pf_norm<8>(float*, const float*, uint32_t, float, _Float16*, float*, const float*, size_t,
+                                      uint32_t*);
+
 // Q/K RMSNorm per head (model.rs:233-238), NeoX RoPE at position p0 + t
 // (ops.rs:16-28), KV append (model.rs:241-243).  Row t of QKV is
 // [q (heads*128) | k (kvheads*128) | v (kvheads*128)].  Q goes to
 // Q16[head][t][128] (fp16), K and V to the fp32 cache [kvhead][ctx][128].
-// Wave w takes head slots w, w + kWaves, ...: 0..heads-1 q, then k, then v;
-// lane l holds elements l and l + 64, the rotated pair.
-__global__ __launch_bounds__(kBlock) void k_pf_qkrope(const float* QKV, const float* qn, const float* kn,
+// Wave w of the token's gridDim.y workgroups takes head slots w, w + waves,
+// ...: 0..heads-1 q, then k, then v; lane l holds elements l and l + 64, the
+// rotated pair.  QKV comes as Z column splits (qstride floats apart), added in
+// split order; a wave requests every split of kSW slots before it adds any.
+template <int Z>
+__global__ __launch_bounds__(kBlock) void k_pf_qkrope(const float* QKV, size_t qstride, const float* qn, const float* kn,
                                                       const float2* rope, uint32_t p0, uint32_t S, uint32_t heads,
                                                       uint32_t kvheads, uint32_t ctx, float eps, _Float16* Q16,
                                                       float* kcache, float* vcache, _Float16* Kh, _Float16* Vth,
                                                       uint32_t vp, uint32_t* err) {
-    const uint32_t t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6, pos = p0 + t;
+    const uint32_t t = blockIdx.x, lane = threadIdx.x & 63, pos = p0 + t;
+    const uint32_t nw = gridDim.y * kWaves, w = blockIdx.y * kWaves + (threadIdx.x >> 6);
     const uint32_t row = (heads + 2 * kvheads) * 128;
     const float* x = QKV + (size_t)t * row;
     const float2 cs = rope[(size_t)pos * 64 + lane];
     const uint32_t nslot = heads + 2 * kvheads;
     const float qw0 = qn[lane], qw1 = qn[lane + 64], kw0 = kn[lane], kw1 = kn[lane + 64];
-    constexpr uint32_t kSW = 5;  // slots per wave per round, their loads issued together
+    constexpr uint32_t kSW = qkrope_slots(Z);  // slots per wave per round, their loads issued together
     bool bad = false;
-    for (uint32_t s0 = w; s0 < nslot; s0 += kSW * kWaves) {  // wave-uniform
-        float xa_[kSW], xb_[kSW];
+    for (uint32_t s0 = w; s0 < nslot; s0 += kSW * nw) {  // wave-uniform
+        float xa_[kSW], xb_[kSW], pa[kSW][Z], pb[kSW][Z];
 #pragma unroll
         for (uint32_t j = 0; j < kSW; j++) {
-            const uint32_t sl = min(s0 + j * kWaves, nslot - 1);
-            xa_[j] = x[sl * 128 + lane];
-            xb_[j] = x[sl * 128 + lane + 64];
+            const uint32_t sl = min(s0 + j * nw, nslot - 1);
+#pragma unroll
+            for (int z = 0; z < Z; z++) {
+                pa[j][z] = x[z * qstride + sl * 128 + lane];
+                pb[j][z] = x[z * qstride + sl * 128 + lane + 64];
+            }
         }
 #pragma unroll
         for (uint32_t j = 0; j < kSW; j++) {
-            const uint32_t slot = s0 + j * kWaves;
+            xa_[j] = pa[j][0];
+            xb_[j] = pb[j][0];
+#pragma unroll
+            for (int z = 1; z < Z; z++) {
+                xa_[j] += pa[j][z];
+                xb_[j] += pb[j][z];
+            }
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kSW; j++) {
+            const uint32_t slot = s0 + j * nw;
             if (slot >= nslot) break;
             const float xa = xa_[j], xb = xb_[j];
             if (slot >= heads + kvheads) {
@@ -726,6 +900,19 @@ __global__ __launch_bounds__(kBlock) void k_pf_qkrope(const float* QKV, const fl
     }
     note_range(bad, err);
 }
+
+template __global__ void k_pf_qkrope<1>(const float*, size_t, const float*, const float*, const float2*, uint32_t, uint32_t,
+                                        uint32_t, uint32_t, uint32_t, float, _Float16*, float*, float*, _Float16*,
+                                        _Float16*, uint32_t, uint32_t*);
+template __global__ void k_pf_qkrope<2>(const float*, size_t, const float*, const float*, const float2*, uint32_t, uint32_t,
+                                        uint32_t, uint32_t, uint32_t, float, _Float16*, float*, float*, _Float16*,
+                                        _Float16*, uint32_t, uint32_t*);
+template __global__ void k_pf_qkrope<4>(const float*, size_t, const float*, const float*, const float2*, uint32_t, uint32_t,
+                                        uint32_t, uint32_t, uint32_t, float, _Float16*, float*, float*, _Float16*,
+                                        _Float16*, uint32_t, uint32_t*);
+template __global__ void k_pf_qkrope<8>(const float*, size_t, const float*, const float*, const float2*, uint32_t, uint32_t,
+                                        uint32_t, uint32_t, uint32_t, float, _Float16*, float*, float*, _Float16*,
+                                        _Float16*, uint32_t, uint32_t*);
 
 // Router logits (model.rs:249-256) in fp32 on the matrix cores
 // (v_mfma_f32_16x16x4_f32: fp32 operands and accumulation): 64 tokens per
