@@ -55,6 +55,9 @@ void launch_read_stream(const void*, size_t, uint32_t*, uint32_t, hipStream_t);
 template <uint32_t K>
 __global__ void k_gemm_gateup(const _Float16*, uint32_t, ExpertTiles, DevMat, DevMat, _Float16*, uint32_t*);
 template <uint32_t K> __global__ void k_gemm_down(const _Float16*, ExpertTiles, DevMat, float*);
+template <uint32_t K, int MB>
+__global__ void k_gemm_gateup_skinny(const _Float16*, uint32_t, ExpertTiles, DevMat, DevMat, _Float16*, uint32_t*);
+template <uint32_t K, int MB> __global__ void k_gemm_down_skinny(const _Float16*, ExpertTiles, DevMat, float*);
 __global__ void k_gemm_dense(const _Float16*, uint32_t, DenseSegs, float*, uint32_t, size_t);
 __global__ void k_pf_embed(DevMat, const uint32_t*, uint32_t, uint32_t, float*, DevState*);
 __global__ void k_tile_gemm(DevMat, uint32_t, uint8_t*);
@@ -72,8 +75,8 @@ __global__ void k_pf_kvh(const float*, const float*, uint32_t, uint32_t, uint32_
 __global__ void k_pf_router(const float*, DevMat, uint32_t, uint32_t, uint32_t, float*);
 __global__ void k_pf_topk(const float*, uint32_t, uint32_t, uint32_t, uint32_t*, float*, DevState*, uint32_t*, float*,
                           uint32_t, uint32_t, uint32_t);
-__global__ void k_pf_group(const uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, uint32_t*, uint32_t*,
-                           uint32_t*, uint32_t*);
+__global__ void k_pf_group(const uint32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t*, uint32_t*, uint32_t*,
+                           uint32_t*, uint32_t*, uint32_t*);
 __global__ void k_pf_combine(float*, const float*, const float*, uint32_t, uint32_t, const float*, float, _Float16*,
                              uint32_t*);
 }  // namespace qh
@@ -989,7 +992,7 @@ void prefill_alloc(qh_ctx* c, uint32_t cap) {
     const ModelDims& d = c->dm;
     const uint64_t H = d.hidden, qd = (uint64_t)d.heads * 128, kvd = (uint64_t)d.kvheads * 128;
     const uint64_t n_asg = (uint64_t)cap * d.top;
-    const uint32_t max_tiles = (uint32_t)((n_asg + 127) / 128 + d.experts);
+    const uint32_t max_tiles = (uint32_t)((n_asg + 31) / 32 + d.experts);
     auto up = [](uint64_t b) { return (b + 255) / 256 * 256; };
     const uint64_t npair = ((cap + 15) / 16 + 1) / 2 * d.kvheads;  // attention block pairs
     // a dense launch with more than one column split writes at most
@@ -1124,17 +1127,24 @@ void prefill_layer(qh_ctx* c, size_t l, uint32_t S, uint32_t p0) {
     hipLaunchKernelGGL(k_pf_topk, dim3((S + kWaves - 1) / kWaves), dim3(kBlock), 0, c->s, P.LR, S,
                        d.experts, d.top, P.ids, P.wts, c->acts.st, c->acts.route_log, c->acts.gap_log, d.layers,
                        (uint32_t)l, p0);
-    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, c->s, P.ids, S * d.top, d.top, d.experts, P.goff, P.tok,
+    const uint32_t gm = prefill_tile_rows(S, d.top, d.experts);
+    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, c->s, P.ids, S * d.top, d.top, d.experts, gm, P.goff, P.tok,
                        P.asg, P.te, P.tm, P.ntile);
     const ExpertTiles T{P.goff, P.tok, P.asg, P.te, P.tm, P.ntile};
-    const uint32_t tiles = (S * d.top + 127) / 128 + d.experts;
-    dispatch_km(L.gate.kind, [&](auto K) {
-        hipLaunchKernelGGL(k_gemm_gateup<decltype(K)::value>, dim3(8 * ((tiles + 7) / 8) * ((d.ff + 127) / 128)), dim3(256), 0, c->s,
-                           P.Xn16, H, T, L.gate, L.up, P.Hs, err);
+    const uint32_t tiles = (S * d.top + gm - 1) / gm + d.experts;
+    const uint32_t per_col = 8 * ((tiles + 7) / 8);  // workgroups per column tile (xcd_tile)
+    const dim3 gu(per_col * ((d.ff + 127) / 128)), dn(per_col * ((H + 127) / 128));
+    dispatch_km(L.gate.kind, [&](auto K_) {
+        constexpr uint32_t K = decltype(K_)::value;
+        if (gm == 32) hipLaunchKernelGGL((k_gemm_gateup_skinny<K, 1>), gu, dim3(256), 0, c->s, P.Xn16, H, T, L.gate, L.up, P.Hs, err);
+        else if (gm == 64) hipLaunchKernelGGL((k_gemm_gateup_skinny<K, 2>), gu, dim3(256), 0, c->s, P.Xn16, H, T, L.gate, L.up, P.Hs, err);
+        else hipLaunchKernelGGL(k_gemm_gateup<K>, gu, dim3(256), 0, c->s, P.Xn16, H, T, L.gate, L.up, P.Hs, err);
     });
-    dispatch_km(L.down.kind, [&](auto K) {
-        hipLaunchKernelGGL(k_gemm_down<decltype(K)::value>, dim3(8 * ((tiles + 7) / 8) * ((H + 127) / 128)), dim3(256), 0, c->s, P.Hs, T,
-                           L.down, P.Y);
+    dispatch_km(L.down.kind, [&](auto K_) {
+        constexpr uint32_t K = decltype(K_)::value;
+        if (gm == 32) hipLaunchKernelGGL((k_gemm_down_skinny<K, 1>), dn, dim3(256), 0, c->s, P.Hs, T, L.down, P.Y);
+        else if (gm == 64) hipLaunchKernelGGL((k_gemm_down_skinny<K, 2>), dn, dim3(256), 0, c->s, P.Hs, T, L.down, P.Y);
+        else hipLaunchKernelGGL(k_gemm_down<K>, dn, dim3(256), 0, c->s, P.Hs, T, L.down, P.Y);
     });
     // + the next layer's attention RMSNorm (fp16 operand of its q|k|v GEMM)
     const float* next_norm = l + 1 < c->layers.size() ? c->layers[l + 1].attn_norm : nullptr;

@@ -222,8 +222,21 @@ QH_HD constexpr uint32_t qkrope_slots(uint32_t z) { return z == 1 ? 5 : z == 2 ?
 // block pair and KV head.
 constexpr uint32_t kPfAttnSlot = 4 * 68 * 64;
 
+// Rows of the expert GEMMs' tiles for S tokens, by the mean tokens per expert:
+// 32 while most experts fit one such tile, 64 likewise (a second tile of an
+// expert dequantises its weights again), else 128.  Four 30B layers, us per
+// prefill with 32 / 64 / 128 rows: 24 tokens 674 / 731 / 790; 256 tokens 962 /
+// 1,030 / 1,100; 400 tokens (mean 25) 1,081 / 1,116; 517 (mean 32) 1,222 /
+// 1,200; 900 (mean 56) 1,428 at 64, 1,450 at 128; 1,200 (mean 75) 1,777 / 1,727.
+constexpr uint32_t kPfRows32 = 26, kPfRows64 = 64;
+QH_HD uint32_t prefill_tile_rows(uint32_t S, uint32_t top, uint32_t experts) {
+    const uint32_t mean = S * top / experts;  // tokens per expert
+    return mean <= kPfRows32 ? 32 : mean <= kPfRows64 ? 64 : 128;
+}
+
 // Expert work list of the batched-prefill grouped GEMMs (prefill.hip): tile
-// y covers rows [tm, tm + 128) of expert te; the rows of expert e are
+// y covers rows [tm, tm + gm) of expert te (gm = 128, or 64 or 32 when the
+// experts get few tokens each: prefill_tile_rows); the rows of expert e are
 // [goff[e], goff[e+1]) of the assignments sorted by expert.
 struct ExpertTiles {
     const uint32_t* goff;   // [E + 1]

@@ -374,84 +374,92 @@ __device__ __forceinline__ void gemm_tile_r(const _Float16* const (&arows)[4], c
 
 // The same product for a tile of at most 32 MB rows (MB = 1, 2): a prompt or
 // an expert with few rows.  There the weights' bytes bound the launch, not the
-// products, so the loop is built to keep more of them in flight: a step is one
-// whole 256-column super-block (32 or 64 KB of weights per workgroup requested
-// one step ahead, each row's header once instead of once per slice), the
-// activations of 256 / MB columns are staged per barrier, and the unused row
-// blocks cost no registers.  acc[nb][mb] += A[m0 .. m0 + 32 MB) x
-// W_nb[n0 .. n0+128)^T over super-blocks [sb0, sb0 + nsb); arows[i]: the A row
-// of tile row srow_row<MB>(i) (any valid row past the tile's rows).
+// products, so the loop keeps more of them in flight: WS slices of weights
+// (half a super-block or a whole one) are requested one such group ahead, each
+// row's header once per group, the activations of 256 / MB columns are staged
+// per barrier, and unused row blocks cost no registers.
+// acc[nb][mb] += A[m0 .. m0 + 32 MB) x W_nb[n0 .. n0+128)^T over super-blocks
+// [sb0, sb0 + nsb); arows[i]: the A row of tile row srow_row<MB>(i) (any valid
+// row past the tile's rows).
 constexpr int kSP(int mb) { return 256 / mb + 8; }                 // LDS row pitch in halfs
-constexpr int kRS = 2 * 32 * (256 + 8);                            // halfs of LDS, MB = 1
-constexpr int kRS2 = 2 * 64 * (128 + 8);                           // halfs of LDS, MB = 2
+constexpr int kRS(int mb) { return 2 * 32 * mb * kSP(mb); }        // halfs of LDS: two staged parts
 template <int MB> __device__ __forceinline__ uint32_t srow_row(uint32_t i) {
     return (threadIdx.x + kGT * i) / (32 / MB);  // 32 / MB 16-byte chunks per staged row
 }
-template <uint32_t KIND, int NB, int MB>
+template <uint32_t KIND, int NB, int MB, int WS>
 __device__ __forceinline__ void gemm_skinny(const _Float16* const (&arows)[4], const uint8_t* const (&wblk)[NB],
                                             uint32_t sb0, uint32_t nsb, f16v (&acc)[NB][MB], _Float16* As) {
-    constexpr int KS = 4 / MB, P = kSP(MB);  // slices per staged part, LDS pitch
+    constexpr int KS = 4 / MB, P = kSP(MB), WP = 4 / WS;  // slices per staged part, LDS pitch, weight groups per block
     const uint32_t lane = threadIdx.x & 63, grp = lane >> 5;
     const uint32_t ach = threadIdx.x % (32 / MB);
-    WReg<KIND> wr[2][NB][4];
+    WReg<KIND> wr[2][NB][WS];
     uint4 av[4];
-    auto wload = [&](auto B_, uint32_t i) {
+    auto wload = [&](auto B_, uint32_t i, auto G_) {  // group G of super-block i
         const size_t o = (size_t)(sb0 + min(i, nsb - 1)) * tile_block_bytes(KIND);  // past the end: a harmless reload
 #pragma unroll
         for (int nb = 0; nb < NB; nb++)
 #pragma unroll
-            for (int sl = 0; sl < 4; sl++) wr[decltype(B_)::value][nb][sl].load(wblk[nb] + o, sl, lane);
+            for (int sl = 0; sl < WS; sl++)
+                wr[decltype(B_)::value][nb][sl].load(wblk[nb] + o, WS * decltype(G_)::value + sl, lane);
     };
     auto aload = [&](uint32_t j) {  // staged part j: columns 256 sb0 + 64 KS j ..
         const uint32_t k0 = 256 * sb0 + 64 * KS * min(j, MB * nsb - 1);
 #pragma unroll
         for (int i = 0; i < 4; i++) av[i] = gld<uint4>(arows[i] + k0 + 8 * ach);
     };
+    using I0 = std::integral_constant<int, 0>;
     aload(0);
-    wload(std::integral_constant<int, 0>{}, 0);
-    auto step = [&](auto B_, uint32_t i) {
-        constexpr int B = decltype(B_)::value;
-#pragma unroll
-        for (int part = 0; part < MB; part++) {
-            const uint32_t j = MB * i + part;
-            _Float16* Ab = As + (j & 1) * 32 * MB * P;
+    wload(I0{}, 0, I0{});
+    auto slice = [&](auto SL_, auto B0_, uint32_t i) {
+        constexpr int sl = decltype(SL_)::value, part = sl / KS, ks = sl % KS, wg = sl / WS;
+        constexpr int B = WS == 4 ? decltype(B0_)::value : wg & 1;
+        const uint32_t j = MB * i + part;
+        _Float16* Ab = As + (j & 1) * 32 * MB * P;
+        if constexpr (ks == 0) {
 #pragma unroll
             for (int r = 0; r < 4; r++)
                 *reinterpret_cast<uint4*>(Ab + srow_row<MB>(r) * P + 8 * ach) = av[r];
             aload(j + 1);
-            if (part == 0) wload(std::integral_constant<int, 1 - B>{}, i + 1);
-            __syncthreads();  // the buffer's readers of part j - 2 passed the barrier of part j - 1
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const int sl = KS * part + ks;
-                typename WReg<KIND>::Sc sc[NB];
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++) sc[nb] = wr[B][nb][sl].prep(sl, grp);
-                auto kstep = [&](auto S_) {
-                    constexpr int S = decltype(S_)::value;
-                    const uint32_t col = 64 * ks + 32 * (S >> 1) + 16 * grp + 8 * (S & 1);
-                    h8v af[MB];
-#pragma unroll
-                    for (int mb = 0; mb < MB; mb++)
-                        af[mb] = *reinterpret_cast<const h8v*>(Ab + (32 * mb + (lane & 31)) * P + col);
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++) {
-                        const h8v bf = wr[B][nb][sl].template dequant<S>(sc[nb], sl & 1);
-#pragma unroll
-                        for (int mb = 0; mb < MB; mb++)
-                            acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf, acc[nb][mb], 0, 0, 0);
-                    }
-                };
-                kstep(std::integral_constant<int, 0>{});
-                kstep(std::integral_constant<int, 1>{});
-                kstep(std::integral_constant<int, 2>{});
-                kstep(std::integral_constant<int, 3>{});
-            }
         }
+        if constexpr (sl % WS == 0)
+            wload(std::integral_constant<int, 1 - B>{}, i + (wg + 1) / WP, std::integral_constant<int, (wg + 1) % WP>{});
+        if constexpr (ks == 0) __syncthreads();  // the readers of part j - 2 passed the barrier of part j - 1
+        typename WReg<KIND>::Sc sc[NB];
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) sc[nb] = wr[B][nb][sl % WS].prep(sl, grp);
+        auto kstep = [&](auto S_) {
+            constexpr int S = decltype(S_)::value;
+            const uint32_t col = 64 * ks + 32 * (S >> 1) + 16 * grp + 8 * (S & 1);
+            h8v af[MB];
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++)
+                af[mb] = *reinterpret_cast<const h8v*>(Ab + (32 * mb + (lane & 31)) * P + col);
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+                const h8v bf = wr[B][nb][sl % WS].template dequant<S>(sc[nb], sl & 1);
+#pragma unroll
+                for (int mb = 0; mb < MB; mb++)
+                    acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf, acc[nb][mb], 0, 0, 0);
+            }
+        };
+        kstep(std::integral_constant<int, 0>{});
+        kstep(std::integral_constant<int, 1>{});
+        kstep(std::integral_constant<int, 2>{});
+        kstep(std::integral_constant<int, 3>{});
     };
-    for (uint32_t i = 0; i < nsb; i += 2) {
-        step(std::integral_constant<int, 0>{}, i);
-        if (i + 1 < nsb) step(std::integral_constant<int, 1>{}, i + 1);  // workgroup-uniform
+    auto step = [&](auto B_, uint32_t i) {
+        slice(std::integral_constant<int, 0>{}, B_, i);
+        slice(std::integral_constant<int, 1>{}, B_, i);
+        slice(std::integral_constant<int, 2>{}, B_, i);
+        slice(std::integral_constant<int, 3>{}, B_, i);
+    };
+    if constexpr (WS == 4) {
+        for (uint32_t i = 0; i < nsb; i += 2) {
+            step(I0{}, i);
+            if (i + 1 < nsb) step(std::integral_constant<int, 1>{}, i + 1);  // workgroup-uniform
+        }
+    } else {
+        for (uint32_t i = 0; i < nsb; i++) step(I0{}, i);
     }
 }
 
@@ -544,6 +552,82 @@ __global__ __launch_bounds__(kGT, 2) void k_gemm_down(const _Float16* Hs, Expert
         }
 }
 
+// k_gemm_gateup and k_gemm_down on tiles of 32 MB rows (the work list of a
+// prompt whose experts get few tokens each).  Bound by the experts' weight
+// bytes (226 MB of gate and up rows per layer when every expert is used): at
+// 24 tokens (about 100 experts, 179 MB) gate/up take 41 us per layer, down 21-27
+// us, against 53 and 32-37 us on 128-row tiles.
+template <uint32_t KIND, int MB>
+__global__ __launch_bounds__(kGT, 3 - (MB - 1)) void k_gemm_gateup_skinny(const _Float16* Xn, uint32_t H, ExpertTiles G,
+                                                                          DevMat Wg, DevMat Wu, _Float16* Hs,
+                                                                          uint32_t* err) {
+    __shared__ __align__(16) _Float16 smem[kRS(MB)];
+    uint32_t ty, tx;
+    xcd_tile((Wg.rows + kGN - 1) / kGN, ty, tx);
+    if (ty >= *G.ntile) return;
+    const uint32_t e = G.te[ty], mt0 = G.tm[ty];
+    const uint32_t base = G.goff[e], rows = G.goff[e + 1] - base;
+    const uint32_t n0 = tx * kGN, ff = Wg.rows;
+    const _Float16* arows[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+        arows[i] = Xn + (size_t)G.tok[base + min(mt0 + srow_row<MB>(i), rows - 1)] * H;
+    const size_t gofs = (size_t)min((n0 >> 5) + (threadIdx.x >> 6), ff / 32 - 1) * tile_group_bytes(KIND, Wg.cols);
+    const uint8_t* const wblk[2] = {Wg.wt + e * Wg.expert_stride + gofs, Wu.wt + e * Wu.expert_stride + gofs};
+    f16v acc[2][MB];
+#pragma unroll
+    for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) acc[nb][mb] = f16v{};
+    gemm_skinny<KIND, 2, MB, 2>(arows, wblk, 0, Wg.cols / 256, acc, smem);
+    const uint32_t n = n0 + racc_col();
+    bool bad = false;
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t m = mt0 + racc_row(mb, i);
+            if (m < rows && n < ff) {
+#pragma clang fp contract(off)
+                const float gv = acc[0][mb][i], uv = acc[1][mb][i];
+                Hs[(size_t)(base + m) * ff + n] = to_h((gv / (1.f + expf(-gv))) * uv, bad);
+            }
+        }
+    note_range(bad, err);
+}
+
+template <uint32_t KIND, int MB>
+__global__ __launch_bounds__(kGT, 3) void k_gemm_down_skinny(const _Float16* Hs, ExpertTiles G, DevMat Wd, float* Y) {
+    __shared__ __align__(16) _Float16 smem[kRS(MB)];
+    __shared__ uint32_t dsts[32 * MB];  // assignment index of each tile row
+    uint32_t ty, tx;
+    xcd_tile((Wd.rows + kGN - 1) / kGN, ty, tx);
+    if (ty >= *G.ntile) return;
+    const uint32_t e = G.te[ty], mt0 = G.tm[ty];
+    const uint32_t base = G.goff[e], rows = G.goff[e + 1] - base;
+    const uint32_t n0 = tx * kGN, ff = Wd.cols, N = Wd.rows;
+    // visible to the epilogue through the GEMM's barriers
+    if (threadIdx.x < 32 * MB) dsts[threadIdx.x] = G.asg[base + min(mt0 + threadIdx.x, rows - 1)];
+    const _Float16* arows[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) arows[i] = Hs + (size_t)(base + min(mt0 + srow_row<MB>(i), rows - 1)) * ff;
+    const uint8_t* const wblk[1] = {
+        Wd.wt + e * Wd.expert_stride +
+        (size_t)min((n0 >> 5) + (threadIdx.x >> 6), N / 32 - 1) * tile_group_bytes(KIND, Wd.cols)};
+    f16v acc[1][MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) acc[0][mb] = f16v{};
+    gemm_skinny<KIND, 1, MB, 4>(arows, wblk, 0, ff / 256, acc, smem);
+    const uint32_t n = n0 + racc_col();
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t ml = racc_row(mb, i), m = mt0 + ml;
+            if (m < rows && n < N) Y[(size_t)dsts[ml] * N + n] = acc[0][mb][i];
+        }
+}
+
 // Dense projections (the per-token q/k/v and o matvecs of model.rs:230-232,
 // 245 over a chunk), up to three matrices of either format in one launch so
 // that the small k and v projections share the machine with q:
@@ -626,7 +710,7 @@ __device__ __forceinline__ void dense_skinny_body(const _Float16* X16, uint32_t 
     f16v acc[1][MB];
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) acc[0][mb] = f16v{};
-    gemm_skinny<KIND, 1, MB>(arows, wblk, sb0, nsb, acc, smem);
+    gemm_skinny<KIND, 1, MB, 4>(arows, wblk, sb0, nsb, acc, smem);
     const uint32_t n = n0 + racc_col();
 #pragma unroll
     for (int mb = 0; mb < MB; mb++)
@@ -640,7 +724,7 @@ __device__ __forceinline__ void dense_skinny_body(const _Float16* X16, uint32_t 
 template <int MB>
 __global__ __launch_bounds__(kGT, 2) void k_gemm_dense_skinny(const _Float16* X16, uint32_t S, DenseSegs G, float* C,
                                                               uint32_t ldc, size_t split_stride) {
-    __shared__ __align__(16) _Float16 smem[MB == 1 ? kRS : kRS2];
+    __shared__ __align__(16) _Float16 smem[kRS(MB)];
     const uint32_t t = blockIdx.x;
     const uint32_t i = t < G.tile_end[0] ? 0 : t < G.tile_end[1] ? 1 : 2;  // workgroup-uniform
     const uint32_t t0 = i == 0 ? 0 : G.tile_end[i - 1];
@@ -1078,13 +1162,13 @@ __global__ __launch_bounds__(kBlock) void k_pf_topk(const float* LR, uint32_t S,
 // Groups the S*top (token, slot) assignments by expert (one workgroup):
 // goff = exclusive prefix of the per-expert counts, tok/asg = the
 // assignments sorted by expert (order within an expert is arbitrary), and
-// the list of 128-row GEMM tiles (te, tm).  Up to 16,384 assignments are
+// the list of gm-row GEMM tiles (te, tm).  Up to 16,384 assignments are
 // placed in LDS first and stored in order (coalesced: stored straight to
 // their sorted positions, every store instruction of a wave touched up to 64
 // cache lines).
 __global__ __launch_bounds__(1024) void k_pf_group(const uint32_t* ids, uint32_t n, uint32_t top, uint32_t E,
-                                                   uint32_t* goff, uint32_t* tok, uint32_t* asg, uint32_t* te,
-                                                   uint32_t* tm, uint32_t* ntile) {
+                                                   uint32_t gm, uint32_t* goff, uint32_t* tok, uint32_t* asg,
+                                                   uint32_t* te, uint32_t* tm, uint32_t* ntile) {
     __shared__ uint32_t cnt[256], cur[256], tb[256];  // E <= 255
     __shared__ uint32_t srt[16384], ntot;              // sorted assignments, their count
     for (uint32_t e = threadIdx.x; e < 256; e += 1024) cnt[e] = 0;
@@ -1113,7 +1197,7 @@ __global__ __launch_bounds__(1024) void k_pf_group(const uint32_t* ids, uint32_t
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) {
             c4[k] = cnt[4 * lane + k];  // zero past E
-            t4[k] = (c4[k] + kGM - 1) / kGM;
+            t4[k] = (c4[k] + gm - 1) / gm;
             cs += c4[k];
             ts += t4[k];
         }
@@ -1143,7 +1227,7 @@ __global__ __launch_bounds__(1024) void k_pf_group(const uint32_t* ids, uint32_t
     }
     __syncthreads();
     for (uint32_t e = threadIdx.x; e < E; e += 1024)
-        for (uint32_t m = 0, t = tb[e]; m < cnt[e]; m += kGM, t++) {
+        for (uint32_t m = 0, t = tb[e]; m < cnt[e]; m += gm, t++) {
             te[t] = e;
             tm[t] = m;
         }
@@ -1585,10 +1669,16 @@ __global__ __launch_bounds__(kBlock) void k_pf_kvh(const float* kcache, const fl
     }
 }
 
+#define QH_INSTANTIATE_PREFILL_SKINNY(K, MB)                                                                        \
+    template __global__ void k_gemm_gateup_skinny<K, MB>(const _Float16*, uint32_t, ExpertTiles, DevMat, DevMat,    \
+                                                         _Float16*, uint32_t*);                                     \
+    template __global__ void k_gemm_down_skinny<K, MB>(const _Float16*, ExpertTiles, DevMat, float*);
 #define QH_INSTANTIATE_PREFILL_GEMM(K)                                                                          \
     template __global__ void k_gemm_gateup<K>(const _Float16*, uint32_t, ExpertTiles, DevMat, DevMat, _Float16*,      \
                                               uint32_t*);                                                           \
-    template __global__ void k_gemm_down<K>(const _Float16*, ExpertTiles, DevMat, float*);                          \
+    template __global__ void k_gemm_down<K>(const _Float16*, ExpertTiles, DevMat, float*);                            \
+    QH_INSTANTIATE_PREFILL_SKINNY(K, 1)                                                                             \
+    QH_INSTANTIATE_PREFILL_SKINNY(K, 2)
 
 QH_INSTANTIATE_PREFILL_GEMM(Q4_0)
 QH_INSTANTIATE_PREFILL_GEMM(Q8_0)
