@@ -1223,55 +1223,45 @@ namespace {
 uint32_t run_sample(qh_ctx* c, qh_sampler* sp, const float* dlogits, const uint8_t* dvalid, size_t n) {
     if (n == 0) throw Error("invalid logits");
     if (n > (1u << 20)) throw Error("the device sampler takes at most 1048576 logits");
-    c->samp_out.reserve(32);
-    c->pin.reserve(32);
+    HIP_OK(hipSetDevice(c->device));
+    c->samp_out.reserve(sizeof(SampleState));
+    c->pin.reserve(kSampleHead);
     SampleArgs a{};
     a.logits = dlogits;
     a.valid = dvalid;
     a.n = (uint32_t)n;
-    a.top_k = (uint32_t)std::min<size_t>(sp->top_k, 0xffffffffu);
     a.temperature = sp->temperature;
     a.top_p = sp->top_p;
     a.draw = sp->rng.peek_f32();
-    a.mode = kSampleModeSample;
-    a.out = c->samp_out.as<uint32_t>();
-    HIP_OK(hipSetDevice(c->device));
-    const uint32_t* r = static_cast<const uint32_t*>(c->pin.p);
+    a.st = c->samp_out.as<SampleState>();
+    const SampleState* r = static_cast<const SampleState*>(c->pin.p);  // its first kSampleHead bytes
     auto read_out = [&] {
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(c->pin.p, a.out, 32, hipMemcpyDeviceToHost, c->s));
+        HIP_OK(hipMemcpyAsync(c->pin.p, a.st, kSampleHead, hipMemcpyDeviceToHost, c->s));
         HIP_OK(hipStreamSynchronize(c->s));
+        if (r->bad) throw Error("invalid logits");
     };
-    launch_sample(a, c->s);
-    read_out();
-    if (r[1] == kSampleBadLogits) throw Error("invalid logits");
-    if (r[1] == kSampleSupport) {
-        // more candidates than one workgroup sorts in LDS: collect the P ids at
-        // or above the key of rank P - 1 into HBM, sort them there, fold
-        const uint32_t P = r[3];
-        const unsigned long long theta = ((unsigned long long)r[5] << 32) | r[4];
-        const uint32_t K = (a.top_k > 0 && a.top_k < a.n) ? a.top_k : a.n;
-        uint32_t np = 4096;
-        while (np < P) np <<= 1;
-        c->samp_big.reserve((size_t)np * 8 + (size_t)P * 4 + 64);
-        auto* cand = c->samp_big.as<unsigned long long>();
-        float* prob = reinterpret_cast<float*>(cand + np);
-        uint32_t* cnt = reinterpret_cast<uint32_t*>(prob + P);
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, c->s, cnt, (size_t)1, 0u);
-        launch_sample_collect(a, theta, P, np, cand, cnt, c->s);
-        launch_sample_sort(cand, np, c->s);
-        launch_sample_fold(a, cand, prob, P, K, c->s);
+    const uint32_t K = (uint32_t)(sp->top_k > 0 && sp->top_k < n ? sp->top_k : n);
+    const bool greedy = sp->temperature == 0.f, few = !greedy && K <= kSampleMax;
+    hipLaunchKernelGGL(k_fill_u32, dim3(8), dim3(kBlock), 0, c->s, c->samp_out.as<uint32_t>(),
+                       (few ? kSampleClear : kSampleHead) / 4, 0u);
+    launch_sample_scan(a, few, c->s);
+    if (greedy) {
         read_out();
-        if (r[1] == kSampleRank) {  // ids.last() is the id of rank m - 1, past the candidates
-            a.mode = kSampleModeRank;
-            a.rank = r[2] - 1;
-            launch_sample(a, c->s);
-            read_out();
-        }
+        return ~(uint32_t)r->top;
     }
-    if (r[1] != 0) throw Error("device sampler failed");
-    if (sp->temperature != 0.f) sp->rng.word++;
-    return r[0];
+    if (few) {
+        launch_sample_small(a, K, c->s);
+        read_out();
+    }
+    if (!few || r->status == kSampleSupport) {
+        c->samp_big.reserve(sample_sort_bytes(a.n));
+        launch_sample_full(a, K, c->samp_big.p, c->s);
+        read_out();
+    }
+    if (r->status != 0) throw Error("device sampler failed");
+    sp->rng.word++;
+    return r->id;
 }
 
 }  // namespace

@@ -4,6 +4,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
+
 #include "qh_format.hpp"
 
 namespace qh {
@@ -171,36 +173,39 @@ struct DecodeArgs {
 };
 
 // Device sampler (sample.hip): src/sampling.rs:26-63 over n logits in HBM.
-// Up to kSampleMax candidates are sorted in LDS by one workgroup; more go
-// through a global buffer (collected, bitonic-sorted by grid-wide steps,
-// folded by one workgroup).
+// Up to kSampleMax candidates are sorted in LDS by one workgroup; more ids are
+// radix-sorted in HBM and folded by one workgroup.
 constexpr uint32_t kSampleMax = 4096;  // largest candidate list sorted in LDS
 enum : uint32_t {
-    kSampleBadLogits = 1u,  // empty or non-finite logits ("invalid logits")
-    kSampleSupport = 2u,    // more than kSampleMax candidates: out[3] = P, out[4..5] = key of rank P - 1
-    kSampleInternal = 3u,   // the candidate selection did not yield the expected count
-    kSampleRank = 4u,       // the pick is the id of rank out[2] - 1, beyond the candidates
+    kSampleBadLogits = 1u,  // non-finite logits ("invalid logits")
+    kSampleSupport = 2u,    // more than kSampleMax ids share the last candidate's digits: sort them all
 };
-enum : uint32_t { kSampleModeSample = 0u, kSampleModeRank = 1u };
+// Device state of one draw; the words before cand start at zero.
+struct SampleState {
+    unsigned long long top;  // composite key of the first id: key << 32 | ~id
+    uint32_t bad;            // a logit was not finite
+    uint32_t ncand;          // ids gathered so far
+    uint32_t count;          // ids at or above the digit of rank K - 1
+    uint32_t id, status, kept;  // the draw, kSample* status, ids kept by top-p
+    uint32_t hist[2048];     // ids by the top 11 bits of their key
+    unsigned long long cand[kSampleMax];
+};
+constexpr size_t kSampleHead = 32, kSampleClear = offsetof(SampleState, cand);
 struct SampleArgs {
     const float* logits;   // [n]
     const uint8_t* valid;  // [n] 0 = masked to f32::MIN, or null
-    uint32_t n, top_k;     // top_k 0 = no truncation
+    uint32_t n;
     float temperature, top_p;
     float draw;            // rand's gen::<f32>() for this call (unused at temperature 0)
-    uint32_t mode;         // kSampleModeRank: out[0] = the id of rank `rank` of the sort
-    uint32_t rank;
-    uint32_t* out;         // [8] id, status, kept count, candidate count, key of rank P - 1 (2 words)
+    SampleState* st;
 };
-void launch_sample(const SampleArgs& a, hipStream_t s);
-// The candidates beyond kSampleMax: cand[0, np) = the P composite keys >=
-// theta (in any order), then 0 (np a power of two >= P); cnt a zeroed
-// counter.  Then sorted descending and folded (sampling.rs:43-62) into out.
-void launch_sample_collect(const SampleArgs& a, unsigned long long theta, uint32_t P, uint32_t np,
-                           unsigned long long* cand, uint32_t* cnt, hipStream_t s);
-void launch_sample_sort(unsigned long long* cand, uint32_t np, hipStream_t s);
-void launch_sample_fold(const SampleArgs& a, const unsigned long long* cand, float* prob, uint32_t P, uint32_t K,
-                        hipStream_t s);
+// Finiteness and the first id (st->bad, st->top), and with want_hist st->hist.
+void launch_sample_scan(const SampleArgs& a, bool want_hist, hipStream_t s);
+// After a scan with the histogram: the draw among the K <= kSampleMax first ids.
+void launch_sample_small(const SampleArgs& a, uint32_t K, hipStream_t s);
+// After a scan: the draw among the K first ids, with sample_sort_bytes(n) of workspace.
+size_t sample_sort_bytes(uint32_t n);
+void launch_sample_full(const SampleArgs& a, uint32_t K, void* work, hipStream_t s);
 
 // Column splits of the batched prefill's router logits (prefill.hip:
 // k_pf_router writes one partial sum per split, k_pf_topk adds them in split

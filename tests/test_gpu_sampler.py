@@ -108,3 +108,36 @@ def test_model_sample_after_forward(dev):
     lg = m.forward(tok)
     assert m.sample(engine.Sampler(1, 0.0, 0, 1.0)) == oracle.greedy(np.where(valid == 1, lg, FMIN))
     m.set_valid_tokens(None)
+
+
+def _flat(n):
+    return np.zeros(n, np.float32)
+
+
+def _levels(n):
+    lg = np.zeros(n, np.float32)
+    lg[n // 3:] = -0.6931472
+    lg[n // 2:] = -5.5
+    return lg
+
+
+def _ramp(n):
+    return (np.arange(n, dtype=np.float32) * np.float32(-1e-4))[::-1].copy()
+
+
+def _peak(n):
+    lg = np.random.default_rng(n).normal(0, 2.5, n).astype(np.float32)
+    lg[:5] += 15
+    return lg
+
+
+@pytest.mark.parametrize("shape", [_flat, _levels, _ramp, _peak])
+@pytest.mark.parametrize("n,t,k,p", [(151936, 1.0, 0, 1.0), (151936, 0.7, 0, 0.37), (16385, 1.0, 0, 0.9999),
+                                     (4097, 3.0, 4096, 0.8), (20000, 0.01, 0, 0.5), (2049, 1.0, 17, 1.0),
+                                     (70001, 1.3, 4097, 0.97)])
+def test_sampler_folds(dev, shape, n, t, k, p):
+    """The parallel folds and the radix sort at sums that cross many binades,
+    round to even often (equal probabilities), stop changing early, and cut
+    inside and at the ends of segments: the oracle's ids exactly."""
+    got, want = run_both(dev, shape(n), seed=n + k, t=t, k=k, p=p, steps=8)
+    assert got == want
