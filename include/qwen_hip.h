@@ -142,14 +142,16 @@ int qh_attention(qh_ctx *ctx, const float *q, const float *k, const float *v, si
  * the reference; for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  q, k, v
  * and out are device pointers in qh_attention's layouts; the kernel's chunk
- * partials and counters live in a fixed 1 MiB device array of the library
- * (one per GPU).  Both entry points cap the key chunks per KV head at what
+ * partials and counters live in fixed 1 MiB device areas of the library
+ * (eight per GPU, one per calling stream).  Both entry points cap the key chunks per KV head at what
  * the array holds (a chunk then takes several key tiles), so any history
  * length runs; a shape one chunk of whose partials alone exceeds it
  * (heads x (head_dim + 2) floats > 1 MiB) is refused with an error.  stream NULL:
  * the context's stream, and the call returns when out is written; otherwise
  * the work is enqueued on that HIP stream and the call returns at once.
- * Calls that overlap on one GPU share the array and race. */
+ * Calls on up to eight streams of a GPU may overlap; with more, the stream
+ * that called least recently gives up its area, and calls of the two streams
+ * that overlap race. */
 int qh_attention_noalloc(qh_ctx *ctx, const float *q, const float *k, const float *v, size_t klen,
                          size_t heads, size_t kvheads, size_t d, float *out, void *stream);
 

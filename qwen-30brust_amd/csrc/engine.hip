@@ -34,6 +34,8 @@ template <int R> __global__ void k_matvec(DevMat, const float*, float*, int);
 __global__ void k_route(const float*, uint32_t, uint32_t, uint32_t*, float*, uint32_t*);
 __global__ void k_argmax(const float*, uint32_t, int32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*);
 __global__ void k_attention_api(AttnArgs, uint32_t);
+template <int D> __global__ void k_attention_tile(AttnArgs, uint32_t);
+template <int D> __global__ void k_attention_merge(AttnArgs, uint32_t);
 // Token-step kernels (step.hip).
 // Template argument C: held chunk slots per lane (tile_slots), 0 = general.
 template <int C> __global__ void k_qkv(LayerW, DevMat, Acts, ModelDims, int);
@@ -174,30 +176,58 @@ uint64_t groups_host(uint64_t rows, uint64_t cols, int R) {
 
 // ------------------------------------------------ no-allocation scratch --
 // Device memory of qh_attention_noalloc: the chunk partials
-// [heads][chunks][d+2] and the last-arrival counters [kvheads] of
-// k_attention_api, at most kNoAllocScratchBytes.  Every GPU the library runs
-// on holds its own copy for the life of the process; host code uses only the
-// per-device address that hipGetSymbolAddress returns (the array's name is a
-// host-side stand-in, not a device address).
+// [heads][chunks][d+2] and the last-arrival counters [kvheads] of the
+// attention kernels, at most kNoAllocScratchBytes per call.  Every GPU the
+// library runs on holds kNoAllocSlots such areas for the life of the process,
+// one per stream that calls it, so that calls on different streams do not
+// share one (calls on one stream follow each other).  With more streams than
+// areas, the least recently used area goes to the new stream.  Host code uses
+// only the per-device address that hipGetSymbolAddress returns (the array's
+// name is a host-side stand-in, not a device address).
 namespace {
 constexpr size_t kNoAllocScratchBytes = 1u << 20;
+constexpr int kNoAllocSlots = 8;
 constexpr int kNoAllocMaxDevices = 64;
+struct ScratchSlots {
+    uint8_t* base = nullptr;
+    hipStream_t stream[kNoAllocSlots] = {};
+    uint64_t used[kNoAllocSlots] = {};  // time of the slot's last call, 0 = never
+    uint64_t calls = 0;
+};
 std::mutex g_scratch_mu;
-std::array<void*, kNoAllocMaxDevices> g_scratch_ptr{};
+std::array<ScratchSlots, kNoAllocMaxDevices> g_scratch;
 }  // namespace
-static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) uint8_t scratch[kNoAllocSlots * kNoAllocScratchBytes];
 
 // Resolves this device's copy of `scratch` once per device (called by
 // qh_create with the device current).
 static void noalloc_init(int device) {
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     if (device < 0 || device >= kNoAllocMaxDevices) throw Error("device index beyond the scratch table");
-    if (g_scratch_ptr[device]) return;
+    if (g_scratch[device].base) return;
     void* p = nullptr;
     const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e != hipSuccess || p == nullptr)
         throw Error(std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-    g_scratch_ptr[device] = p;
+    g_scratch[device].base = static_cast<uint8_t*>(p);
+}
+
+// The scratch area of calls on stream s.
+static uint8_t* noalloc_scratch(int device, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    ScratchSlots& S = g_scratch[device];
+    if (!S.base) throw Error("no-allocation scratch is not set up on this device");
+    int slot = 0;
+    for (int i = 0; i < kNoAllocSlots; i++) {
+        if (S.used[i] && S.stream[i] == s) {
+            slot = i;
+            break;
+        }
+        if (S.used[i] < S.used[slot]) slot = i;
+    }
+    S.stream[slot] = s;
+    S.used[slot] = ++S.calls;
+    return S.base + slot * kNoAllocScratchBytes;
 }
 
 struct qh_ctx {
@@ -1625,13 +1655,43 @@ AttnGeo attn_geometry(size_t klen, size_t heads, size_t kvheads, size_t d) {
     return g;
 }
 
+// Launches the attention of `a` (its q, k, v, part, counter and out set): the
+// register-tiled kernels where they apply, else the general one, whose
+// arrival counters are cleared first (by a fill kernel: no memset node in a
+// captured graph).
+static void launch_attention(AttnArgs a, const AttnGeo& geo, size_t heads, size_t kvheads, size_t d, hipStream_t s) {
+    a.sh = d;
+    a.st = kvheads * d;
+    a.heads = (uint32_t)heads;
+    a.kvheads = (uint32_t)kvheads;
+    a.d = (uint32_t)d;
+    a.tc = geo.tc;
+    a.max_chunks = geo.nch;
+    a.span = geo.span;
+    a.err = nullptr;
+    const uint32_t T = (uint32_t)geo.T;
+    const bool aligned = ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) % 16 == 0;
+    const dim3 grid((uint32_t)kvheads, geo.nch);
+    if (aligned && (d == 128 || d == 64) && heads / kvheads <= 8) {
+        if (d == 128) {
+            hipLaunchKernelGGL(k_attention_tile<128>, grid, dim3(kBlock), 0, s, a, T);
+            hipLaunchKernelGGL(k_attention_merge<128>, dim3(a.heads), dim3(kBlock), 0, s, a, geo.nch);
+        } else {
+            hipLaunchKernelGGL(k_attention_tile<64>, grid, dim3(kBlock), 0, s, a, T);
+            hipLaunchKernelGGL(k_attention_merge<64>, dim3(a.heads), dim3(kBlock), 0, s, a, geo.nch);
+        }
+    } else {
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, s, a.counter, kvheads, 0u);
+        hipLaunchKernelGGL(k_attention_api, grid, dim3(kBlock), geo.lds, s, a, T);
+    }
+    HIP_OK(hipGetLastError());
+}
+
 int qh_attention(qh_ctx* c, const float* q, const float* k, const float* v, size_t klen, size_t heads,
                  size_t kvheads, size_t d, float* out) {
     return guarded(c, [&] {
         const AttnGeo geo = attn_geometry(klen, heads, kvheads, d);
-        const size_t T = geo.T;
-        const uint32_t tc = geo.tc, nch = geo.nch;
-        auto lds = [&](uint32_t) { return geo.lds; };
+        const uint32_t nch = geo.nch;
         const float* qd = upload_x(c, c->sa, q, heads * d);
         c->sb.reserve(klen * 8 + 256);
         HIP_OK(hipMemcpyAsync(c->sb.p, k, klen * 4, hipMemcpyHostToDevice, c->s));
@@ -1642,25 +1702,14 @@ int qh_attention(qh_ctx* c, const float* q, const float* k, const float* v, size
         float* dpart = c->sc.as<float>();
         float* dout = dpart + part;
         uint32_t* cnt = reinterpret_cast<uint32_t*>(dout + heads * d);
-        HIP_OK(hipMemsetAsync(cnt, 0, kvheads * 4, c->s));
         AttnArgs a{};
         a.q = qd;
         a.k = c->sb.as<float>();
         a.v = c->sb.as<float>() + klen;
-        a.sh = d;
-        a.st = kvheads * d;
-        a.heads = (uint32_t)heads;
-        a.kvheads = (uint32_t)kvheads;
-        a.d = (uint32_t)d;
-        a.tc = tc;
-        a.max_chunks = nch;
-        a.span = geo.span;
         a.part = dpart;
         a.counter = cnt;
         a.out = dout;
-        a.err = nullptr;
-        hipLaunchKernelGGL(k_attention_api, dim3((uint32_t)kvheads, nch), dim3(kBlock), lds(tc), c->s, a, (uint32_t)T);
-        HIP_OK(hipGetLastError());
+        launch_attention(a, geo, heads, kvheads, d, c->s);
         HIP_OK(hipMemcpyAsync(out, dout, heads * d * 4, hipMemcpyDeviceToHost, c->s));
         sync(c);
     });
@@ -1676,31 +1725,17 @@ int qh_attention_noalloc(qh_ctx* c, const float* q, const float* k, const float*
             throw Error("attention over " + std::to_string(geo.T) + " keys needs " + std::to_string(need) +
                         " bytes of scratch; the no-allocation entry point holds " +
                         std::to_string(kNoAllocScratchBytes));
-        uint8_t* base = static_cast<uint8_t*>(g_scratch_ptr[c->device]);
-        if (!base) throw Error("no-allocation scratch is not set up on this device");
-        uint32_t* cnt = reinterpret_cast<uint32_t*>(base + part_bytes);
         hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->s;
-        // the counters start at zero (a fill kernel, no memset node)
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, s, cnt, kvheads, 0u);
+        uint8_t* base = noalloc_scratch(c->device, s);
+        uint32_t* cnt = reinterpret_cast<uint32_t*>(base + part_bytes);
         AttnArgs a{};
         a.q = q;
         a.k = k;
         a.v = v;
-        a.sh = d;
-        a.st = kvheads * d;
-        a.heads = (uint32_t)heads;
-        a.kvheads = (uint32_t)kvheads;
-        a.d = (uint32_t)d;
-        a.tc = geo.tc;
-        a.max_chunks = geo.nch;
-        a.span = geo.span;
         a.part = reinterpret_cast<float*>(base);
         a.counter = cnt;
         a.out = out;
-        a.err = nullptr;
-        hipLaunchKernelGGL(k_attention_api, dim3((uint32_t)kvheads, geo.nch), dim3(kBlock), geo.lds, s, a,
-                           (uint32_t)geo.T);
-        HIP_OK(hipGetLastError());
+        launch_attention(a, geo, heads, kvheads, d, s);
         if (!stream) HIP_OK(hipStreamSynchronize(s));
     });
 }

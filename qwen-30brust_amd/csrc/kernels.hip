@@ -233,4 +233,167 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, uint32_t T) {
 
 __global__ __launch_bounds__(kBlock) void k_attention_api(AttnArgs a, uint32_t T) { attention_block(a, T); }
 
+// The same for head_dim D = 128 or 64, at most 8 query heads per KV head and
+// 16-byte aligned q, k, v (k_attention_api reads single floats, any shape).
+// Bound by latency: at 3,581 keys the 14.7 MB of K and V are 2.3 us of HBM
+// time, spread over one workgroup per CU.  So a workgroup requests a whole
+// 64-key tile of K and V (and its q) at once, with 16-byte loads, and keeps
+// them in registers; eight lanes share a key's dot products with the (up to)
+// eight heads and exchange partial sums in 7 lane steps; a head's softmax is
+// one wave over the tile's keys; each wave adds its own 16 keys to all heads'
+// outputs.  The chunks are merged by a second launch with a workgroup per head
+// (k_attention_merge): merged by the last workgroup of each KV head, four
+// workgroups read all the partials.  32 / 4 heads of 128, 3,581 keys, both
+// launches: 71-119 -> 8 us a call back to back (tile 8.2, merge 3.9 us alone).
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_attention_tile(AttnArgs a, uint32_t T) {
+    constexpr int NQ = D / 32, NV = D / 64;  // float4s of a key's row per lane, dims per lane of a V row
+    constexpr uint32_t kTile = 64, kPW = 16;  // keys per tile, per wave
+    __shared__ float sc[8][kTile + 1];        // scores
+    __shared__ __align__(16) float ps[kTile][8];  // probabilities
+    __shared__ float al[8], red[kWaves][8][D];
+    const uint32_t g = blockIdx.x, ch = blockIdx.y, G = a.heads / a.kvheads;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, kl = lane >> 3, p = lane & 7;
+    const uint32_t k0 = ch * a.span, k1 = min(T, k0 + a.span);
+    if (k0 >= T) return;
+    const float* kb = a.k + (size_t)g * a.sh;
+    const float* vb = a.v + (size_t)g * a.sh;
+    float4 q[8][NQ];
+#pragma unroll
+    for (int h = 0; h < 8; h++)
+#pragma unroll
+        for (int i = 0; i < NQ; i++)
+            q[h][i] = gld<float4>(a.q + (size_t)(g * G + min((uint32_t)h, G - 1)) * D + 4 * (p + 8 * i));
+    float acc[8][NV];
+#pragma unroll
+    for (int h = 0; h < 8; h++)
+#pragma unroll
+        for (int i = 0; i < NV; i++) acc[h][i] = 0.f;
+    const float root = sqrtf((float)D);
+    float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};  // of heads 2 wv and 2 wv + 1
+    for (uint32_t t0 = k0; t0 < k1; t0 += kTile) {
+        float4 kr[2][NQ];
+        float vr[kPW][NV];
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int i = 0; i < NQ; i++)
+                kr[r][i] = gld<float4>(kb + (size_t)min(t0 + kPW * wv + 8 * r + kl, k1 - 1) * a.st + 4 * (p + 8 * i));
+#pragma unroll
+        for (uint32_t j = 0; j < kPW; j++) {  // keys past the end: the last key again, with probability 0
+            const float* row = vb + (size_t)min(t0 + kPW * wv + j, k1 - 1) * a.st;
+            if constexpr (NV == 2) {
+                const float2 t = gld<float2>(row + 2 * lane);
+                vr[j][0] = t.x;
+                vr[j][1] = t.y;
+            } else {
+                vr[j][0] = gld<float>(row + lane);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            float s[8];
+#pragma unroll
+            for (int h = 0; h < 8; h++) {
+                s[h] = 0.f;
+#pragma unroll
+                for (int i = 0; i < NQ; i++) {
+                    s[h] = fmaf(q[h][i].x, kr[r][i].x, s[h]);
+                    s[h] = fmaf(q[h][i].y, kr[r][i].y, s[h]);
+                    s[h] = fmaf(q[h][i].z, kr[r][i].z, s[h]);
+                    s[h] = fmaf(q[h][i].w, kr[r][i].w, s[h]);
+                }
+            }
+            // sums over the key's eight lanes; lane p ends with head p's
+#pragma unroll
+            for (int o = 4; o > 0; o >>= 1) {
+                const bool up = p & o;
+#pragma unroll
+                for (int h = 0; h < o; h++) {
+                    const float keep = up ? s[h + o] : s[h], send = up ? s[h] : s[h + o];
+                    s[h] = keep + __shfl_xor(send, o, 64);
+                }
+            }
+            sc[p][kPW * wv + 8 * r + kl] = s[0];
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t i = 0; i < 2; i++) {
+            const uint32_t h = 2 * wv + i;
+            const float v = t0 + lane < k1 ? sc[h][lane] / root : -INFINITY;
+            const float M = fmaxf(m[i], wave_max(v)), e = expf(v - M), alpha = expf(m[i] - M);  // 0 on the first tile
+            l[i] = fmaf(l[i], alpha, wave_sum(e));
+            m[i] = M;
+            ps[lane][h] = e;
+            if (lane == 0) al[h] = alpha;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 8; h++)
+#pragma unroll
+            for (int i = 0; i < NV; i++) acc[h][i] *= al[h];
+#pragma unroll
+        for (uint32_t j = 0; j < kPW; j++) {
+            const float4 pa = *reinterpret_cast<const float4*>(&ps[kPW * wv + j][0]),
+                         pb = *reinterpret_cast<const float4*>(&ps[kPW * wv + j][4]);
+            const float w[8] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
+#pragma unroll
+            for (int h = 0; h < 8; h++)
+#pragma unroll
+                for (int i = 0; i < NV; i++) acc[h][i] = fmaf(w[h], vr[j][i], acc[h][i]);
+        }
+        // the next tile's scores go to sc, read before the barrier above; its
+        // probabilities are written after the next barrier
+    }
+#pragma unroll
+    for (int h = 0; h < 8; h++)
+#pragma unroll
+        for (int i = 0; i < NV; i++) red[wv][h][NV * lane + i] = acc[h][i];
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < G * D; i += kBlock) {
+        const uint32_t h = i / D, j = i % D;
+        a.part[((size_t)(g * G + h) * a.max_chunks + ch) * (D + 2) + 2 + j] =
+            (red[0][h][j] + red[1][h][j]) + (red[2][h][j] + red[3][h][j]);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 2; i++) {
+        const uint32_t h = 2 * wv + i;
+        if (lane < 2 && h < G)
+            a.part[((size_t)(g * G + h) * a.max_chunks + ch) * (D + 2) + lane] = lane ? l[i] : m[i];
+    }
+}
+
+// out[h] = the merge of head h's nch <= 64 chunk partials (m, l, o).
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_attention_merge(AttnArgs a, uint32_t nch) {
+    constexpr uint32_t NG = kBlock / D;  // chunks taken in turn by NG groups of D threads
+    __shared__ float w[64], red[NG][D];
+    const uint32_t lane = threadIdx.x & 63, j = threadIdx.x % D, grp = threadIdx.x / D;
+    const float* base = a.part + (size_t)blockIdx.x * a.max_chunks * (D + 2);
+    const bool ok = lane < nch;
+    const float* mine = base + (size_t)min(lane, nch - 1) * (D + 2);
+    const float mc = ok ? mine[0] : -INFINITY, lc = ok ? mine[1] : 0.f;
+    constexpr uint32_t kPer = 64 / NG;
+    float o[kPer];
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; i++) o[i] = base[(size_t)min(grp + NG * i, nch - 1) * (D + 2) + 2 + j];
+    const float M = wave_max(mc), e = ok ? expf(mc - M) : 0.f, L = wave_sum(lc * e);
+    if (threadIdx.x < 64) w[lane] = e;
+    __syncthreads();
+    float O = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; i++)
+        if (grp + NG * i < nch) O = fmaf(w[grp + NG * i], o[i], O);
+    red[grp][j] = O;
+    __syncthreads();
+    if (grp == 0) {
+        for (uint32_t k = 1; k < NG; k++) O += red[k][j];
+        a.out[(size_t)blockIdx.x * D + j] = O / L;
+    }
+}
+template __global__ void k_attention_tile<64>(AttnArgs, uint32_t);
+template __global__ void k_attention_tile<128>(AttnArgs, uint32_t);
+template __global__ void k_attention_merge<64>(AttnArgs, uint32_t);
+template __global__ void k_attention_merge<128>(AttnArgs, uint32_t);
+
 }  // namespace qh

@@ -139,3 +139,57 @@ def test_noalloc_refuses_shapes_beyond_its_scratch(dev):
     # the array is left in a usable state
     q, k, v = inputs(32, 64, 8, 2, 64)
     assert np.array_equal(noalloc(dev, q, k, v, 8, 2, 64), dev.attention(q, k, v, 8, 2, 64))
+
+
+def exact(q, k, v, T, heads, kvheads, d):
+    kk = k.reshape(T, kvheads, d).astype(np.float64).repeat(heads // kvheads, 1)
+    vv = v.reshape(T, kvheads, d).astype(np.float64).repeat(heads // kvheads, 1)
+    s = np.einsum("thd,hd->ht", kk, q.reshape(heads, d).astype(np.float64)) / np.sqrt(d)
+    e = np.exp(s - s.max(1, keepdims=True))
+    return np.einsum("ht,thd->hd", e / e.sum(1, keepdims=True), vv)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("heads,kvheads", [(32, 4), (5, 1), (3, 3), (14, 2), (18, 2)])
+@pytest.mark.parametrize("T", [1, 31, 33, 64, 65, 257, 4097])
+def test_attention_shapes(dev, T, heads, kvheads, d):
+    """One to nine query heads per KV head (up to eight: the register-tiled
+    kernel), at tile and chunk edges: within 1e-5 of float64 (32-bit dots of
+    d terms and sums of T weights), and the same bits from both entry points.
+    The same inputs one float off 16-byte alignment run the general kernel."""
+    q, k, v = inputs(T + heads, T, heads, kvheads, d)
+    ref = exact(q, k, v, T, heads, kvheads, d)
+    got = noalloc(dev, q, k, v, heads, kvheads, d)
+    assert np.max(np.abs(got.reshape(heads, d) - ref)) <= 1e-5 * np.max(np.abs(ref))
+    assert np.array_equal(got, dev.attention(q, k, v, heads, kvheads, d))
+    bufs = [DeviceBuffer(np.concatenate([np.zeros(1, np.float32), a])) for a in (q, k, v)]
+    out = DeviceBuffer(np.full(heads * d, np.nan, np.float32))
+    rc = engine.lib().qh_attention_noalloc(dev.h, *[b.ptr.value + 4 for b in bufs], k.size, heads, kvheads, d,
+                                           out.ptr, None)
+    assert rc == 0
+    off = out.read()
+    assert np.max(np.abs(off.reshape(heads, d) - ref)) <= 1e-5 * np.max(np.abs(ref))
+    for b in bufs + [out]:
+        b.free()
+
+
+def test_noalloc_calls_on_several_streams(dev):
+    """Calls queued on four streams without a wait between them (each stream
+    has its own scratch area): every output is the blocking call's."""
+    shape = (32, 4, 128)
+    data = [inputs(50 + i, 900 + 700 * i, *shape) for i in range(4)]
+    want = [noalloc(dev, *d, *shape) for d in data]
+    bufs = [[DeviceBuffer(a) for a in d] + [DeviceBuffer(np.zeros(32 * 128, np.float32))] for d in data]
+    streams = [C.c_void_p() for _ in data]
+    for s in streams:
+        hip_check(hip().hipStreamCreate(C.byref(s)))
+    for _ in range(3):
+        for (q, k, v, out), d, s in zip(bufs, data, streams):
+            assert engine.lib().qh_attention_noalloc(dev.h, q.ptr, k.ptr, v.ptr, d[1].size, *shape, out.ptr, s) == 0
+    for s in streams:
+        hip_check(hip().hipStreamSynchronize(s))
+        hip_check(hip().hipStreamDestroy(s))
+    for b, w in zip(bufs, want):
+        assert np.array_equal(b[3].read(), w)
+        for x in b:
+            x.free()
