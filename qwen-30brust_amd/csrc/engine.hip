@@ -29,6 +29,8 @@ namespace qh {
 __global__ void k_repack(const uint8_t*, uint8_t*, uint32_t, uint32_t, size_t, size_t, size_t);
 __global__ void k_dequant(DevMat, size_t, size_t, float*);
 __global__ void k_fill_u32(uint32_t*, size_t, uint32_t);
+__global__ void k_stage(uint32_t*, const uint32_t*, uint32_t, uint32_t);
+__global__ void k_put_state(DevState*, uint32_t, uint32_t, uint32_t*, uint32_t);
 __global__ void k_router_fold(DevMat, const float*, const float*, uint32_t, uint32_t, uint32_t, float*);
 template <int R> __global__ void k_matvec(DevMat, const float*, float*, int);
 __global__ void k_route(const float*, uint32_t, uint32_t, uint32_t*, float*, uint32_t*);
@@ -137,7 +139,7 @@ struct HostPinned {
         if (p && n >= bytes) return;
         if (p) (void)hipHostFree(p);
         p = nullptr;
-        HIP_OK(hipHostMalloc(&p, bytes));
+        HIP_OK(hipHostMalloc(&p, bytes, hipHostMallocMapped | hipHostMallocCoherent));
         n = bytes;
     }
 };
@@ -298,7 +300,15 @@ struct qh_ctx {
 
     // scratch for the API surfaces
     DevBuf sa, sb, sc, sd;
+    // transfers of the current call through pinned host memory (copy_in,
+    // copy_out): bytes in use, and the caller's buffers to fill after the sync
+    struct Out {
+        void* dst;
+        size_t off, bytes;
+    };
     HostPinned pin;
+    size_t pin_used = 0;
+    std::vector<Out> outs;
 
     // sampler: the padding-vocab mask of the loaded model, host-logits upload
     // buffers and the result words
@@ -342,6 +352,11 @@ thread_local std::string g_create_err;
 
 template <class F> int guarded(qh_ctx* c, F f) {
     try {
+        if (c && c->pin_used) {  // a call that failed before its sync: its copies end, its outputs are dropped
+            (void)hipStreamSynchronize(c->s);
+            c->pin_used = 0;
+            c->outs.clear();
+        }
         f();
         return 0;
     } catch (const std::exception& e) {
@@ -350,7 +365,60 @@ template <class F> int guarded(qh_ctx* c, F f) {
     }
 }
 
-void sync(qh_ctx* c) { HIP_OK(hipStreamSynchronize(c->s)); }
+// Waits for the stream, then hands out what copy_out staged.
+void sync(qh_ctx* c) {
+    const hipError_t e = hipStreamSynchronize(c->s);
+    const std::vector<qh_ctx::Out> outs = std::move(c->outs);
+    c->outs.clear();
+    c->pin_used = 0;
+    HIP_OK(e);
+    for (const auto& o : outs) std::memcpy(o.dst, static_cast<const uint8_t*>(c->pin.p) + o.off, o.bytes);
+}
+
+// Device words copied (and dst zero-filled up to `padded`) by a kernel in the
+// stream; either side may be pinned host memory.
+void launch_stage(qh_ctx* c, void* dst, const void* src, size_t words, size_t padded) {
+    const uint32_t grid = (uint32_t)std::min<size_t>((padded / 4 + kBlock) / kBlock, 256);
+    hipLaunchKernelGGL(k_stage, dim3(grid), dim3(kBlock), 0, c->s, static_cast<uint32_t*>(dst),
+                       static_cast<const uint32_t*>(src), (uint32_t)words, (uint32_t)padded);
+    HIP_OK(hipGetLastError());
+}
+
+// Room for `bytes` in the pinned area until the next sync, or null when this
+// call's transfers do not fit (they then go through hipMemcpyAsync).
+constexpr size_t kPinBytes = 4u << 20;
+uint8_t* pin_room(qh_ctx* c, size_t bytes) {
+    const size_t need = (bytes + 255) / 256 * 256;
+    if (c->pin_used + need > kPinBytes) return nullptr;
+    c->pin.reserve(kPinBytes);
+    uint8_t* p = static_cast<uint8_t*>(c->pin.p) + c->pin_used;
+    c->pin_used += need;
+    return p;
+}
+
+// Caller memory to the device, dst zero-filled up to `padded` bytes; whole
+// 32-bit words are written.
+void copy_in(qh_ctx* c, void* dst, const void* src, size_t bytes, size_t padded = 0) {
+    padded = std::max((bytes + 3) / 4 * 4, padded);
+    if (padded == 0) return;
+    if (uint8_t* p = pin_room(c, bytes)) {
+        std::memcpy(p, src, bytes);
+        launch_stage(c, dst, p, (bytes + 3) / 4, padded / 4);
+        return;
+    }
+    if (padded > bytes) HIP_OK(hipMemsetAsync(static_cast<uint8_t*>(dst) + bytes / 4 * 4, 0, padded - bytes / 4 * 4, c->s));
+    HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->s));
+}
+
+// Device memory (whole words) to the caller's, there after the next sync(c).
+void copy_out(qh_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (uint8_t* p = pin_room(c, bytes)) {
+        launch_stage(c, p, src, bytes / 4, bytes / 4);
+        c->outs.push_back({dst, (size_t)(p - static_cast<uint8_t*>(c->pin.p)), bytes});
+        return;
+    }
+    HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->s));
+}
 
 // Uploads `rows` packed GGUF rows (src) into device rows at dst, repacking on
 // the device through a staging buffer.
@@ -407,8 +475,7 @@ int pick_r(uint64_t rows, uint64_t cols) {
 const float* upload_x(qh_ctx* c, DevBuf& b, const float* x, size_t n) {
     size_t np = pad32h(n);
     b.reserve(np * 4);
-    HIP_OK(hipMemsetAsync(b.p, 0, np * 4, c->s));
-    if (n) HIP_OK(hipMemcpyAsync(b.p, x, n * 4, hipMemcpyHostToDevice, c->s));
+    copy_in(c, b.p, x, n * 4, np * 4);
     c->stats.uploaded_bytes += n * 4;
     return b.as<const float>();
 }
@@ -915,17 +982,17 @@ void need_logits_room(const qh_ctx* c, const float* logits, size_t cap) {
                     std::to_string(c->cfg.vocab));
 }
 
-// Writes the device step state from the host mirror.
-void put_state(qh_ctx* c, uint32_t pos, uint32_t n_given) {
-    DevState st{};
-    st.pos = pos;
-    st.n_given = n_given;
-    HIP_OK(hipMemcpyAsync(c->acts.st, &st, sizeof st, hipMemcpyHostToDevice, c->s));
+// Writes the device step state from the host mirror, and with `token` its
+// token at position pos.
+void put_state(qh_ctx* c, uint32_t pos, uint32_t n_given, const uint32_t* token = nullptr) {
+    hipLaunchKernelGGL(k_put_state, dim3(1), dim3(64), 0, c->s, c->acts.st, pos, n_given,
+                       token ? c->acts.tokens + pos : nullptr, token ? *token : 0u);
+    HIP_OK(hipGetLastError());
 }
 
 DevState get_state(qh_ctx* c) {
     DevState st{};
-    HIP_OK(hipMemcpyAsync(&st, c->acts.st, sizeof st, hipMemcpyDeviceToHost, c->s));
+    copy_out(c, &st, c->acts.st, sizeof st);
     sync(c);
     return st;
 }
@@ -1255,7 +1322,6 @@ uint32_t run_sample(qh_ctx* c, qh_sampler* sp, const float* dlogits, const uint8
     if (n > (1u << 20)) throw Error("the device sampler takes at most 1048576 logits");
     HIP_OK(hipSetDevice(c->device));
     c->samp_out.reserve(sizeof(SampleState));
-    c->pin.reserve(kSampleHead);
     SampleArgs a{};
     a.logits = dlogits;
     a.valid = dvalid;
@@ -1264,11 +1330,16 @@ uint32_t run_sample(qh_ctx* c, qh_sampler* sp, const float* dlogits, const uint8
     a.top_p = sp->top_p;
     a.draw = sp->rng.peek_f32();
     a.st = c->samp_out.as<SampleState>();
-    const SampleState* r = static_cast<const SampleState*>(c->pin.p);  // its first kSampleHead bytes
+    struct Head {  // SampleState's first kSampleHead bytes
+        unsigned long long top;
+        uint32_t bad, ncand, count, id, status, kept;
+    } head{};
+    static_assert(sizeof(Head) == kSampleHead);
+    const Head* r = &head;
     auto read_out = [&] {
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(c->pin.p, a.st, kSampleHead, hipMemcpyDeviceToHost, c->s));
-        HIP_OK(hipStreamSynchronize(c->s));
+        copy_out(c, &head, a.st, kSampleHead);
+        sync(c);
         if (r->bad) throw Error("invalid logits");
     };
     const uint32_t K = (uint32_t)(sp->top_k > 0 && sp->top_k < n ? sp->top_k : n);
@@ -1394,9 +1465,9 @@ int qh_set_valid_tokens(qh_ctx* c, const uint8_t* valid, size_t n) {
         }
         if (n != c->cfg.vocab) throw Error("valid-token mask length differs from the vocabulary");
         HIP_OK(hipSetDevice(c->device));
-        c->valid.reserve(n);
-        HIP_OK(hipMemcpyAsync(c->valid.p, valid, n, hipMemcpyHostToDevice, c->s));
-        HIP_OK(hipStreamSynchronize(c->s));
+        c->valid.reserve(n + 4);
+        copy_in(c, c->valid.p, valid, n);
+        sync(c);
         c->valid_n = n;
     });
 }
@@ -1415,10 +1486,10 @@ int qh_sample_logits(qh_ctx* c, qh_sampler* sp, const float* logits, const uint8
         if (n == 0) throw Error("invalid logits");
         HIP_OK(hipSetDevice(c->device));
         c->samp_logits.reserve(n * 4);
-        HIP_OK(hipMemcpyAsync(c->samp_logits.p, logits, n * 4, hipMemcpyHostToDevice, c->s));
+        copy_in(c, c->samp_logits.p, logits, n * 4);
         if (valid) {
-            c->samp_valid.reserve(n);
-            HIP_OK(hipMemcpyAsync(c->samp_valid.p, valid, n, hipMemcpyHostToDevice, c->s));
+            c->samp_valid.reserve(n + 4);
+            copy_in(c, c->samp_valid.p, valid, n);
         }
         *out = run_sample(c, sp, c->samp_logits.as<float>(), valid ? c->samp_valid.as<uint8_t>() : nullptr, n);
     });
@@ -1502,7 +1573,7 @@ int qh_matvec(qh_ctx* c, const char* name, int64_t expert, const float* x, size_
         const float* xd = upload_x(c, c->sb, x, cols);
         c->sc.reserve((size_t)m.rows * 4);
         launch_matvec(c, m, xd, c->sc.as<float>(), pick_r(m.rows, m.cols));
-        HIP_OK(hipMemcpyAsync(y, c->sc.p, (size_t)m.rows * 4, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, y, c->sc.p, (size_t)m.rows * 4);
         sync(c);
         c->stats.matvecs += 1;
         c->stats.matvec_ms += now_ms() - t0;
@@ -1528,7 +1599,7 @@ int qh_packed_matvec(qh_ctx* c, const void* data, size_t len, uint32_t kind, siz
         const float* xd = upload_x(c, c->sb, x, cols);
         c->sc.reserve(rows * 4);
         launch_matvec(c, m, xd, c->sc.as<float>(), pick_r(rows, cols));
-        HIP_OK(hipMemcpyAsync(y, c->sc.p, rows * 4, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, y, c->sc.p, rows * 4);
         sync(c);
         c->stats.matvecs += 1;
         c->stats.matvec_ms += now_ms() - t0;
@@ -1555,7 +1626,7 @@ int qh_packed_matvec_batch(qh_ctx* c, const void* data, size_t len, uint32_t kin
             throw Error("batched matvec shape not covered (block-quantised rows of <= 8192 columns, "
                         "<= 12288 x floats)");
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(y, c->sc.p, nvec * rows * 4, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, y, c->sc.p, nvec * rows * 4);
         sync(c);
         c->stats.matvecs += nvec;
         c->stats.matvec_ms += now_ms() - t0;
@@ -1575,7 +1646,7 @@ int qh_dequant(qh_ctx* c, const void* data, size_t len, uint32_t kind, size_t ro
         uint32_t grid = (uint32_t)std::min<uint64_t>((rows * cols + kBlock - 1) / kBlock, 65535);
         hipLaunchKernelGGL(k_dequant, dim3(grid), dim3(kBlock), 0, c->s, m, (size_t)0, rows, c->sc.as<float>());
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(out, c->sc.p, rows * cols * 4, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, out, c->sc.p, rows * cols * 4);
         sync(c);
     });
 }
@@ -1589,16 +1660,16 @@ int qh_route(qh_ctx* c, const float* logits, size_t n, size_t top, uint32_t* ids
         uint32_t* dids = c->sc.as<uint32_t>();
         float* dw = reinterpret_cast<float*>(dids + pad32h(top));
         uint32_t* derr = reinterpret_cast<uint32_t*>(dw + pad32h(top));
-        HIP_OK(hipMemsetAsync(derr, 0, 4, c->s));
+        clear_words(c, derr, 4);
         hipLaunchKernelGGL(k_route, dim3(1), dim3(kBlock), top * 4, c->s, ld, (uint32_t)n, (uint32_t)top, dids, dw, derr);
         HIP_OK(hipGetLastError());
-        uint32_t e = 0;
-        HIP_OK(hipMemcpyAsync(&e, derr, 4, hipMemcpyDeviceToHost, c->s));
+        // ids, weights and the error word are one run of words
+        std::vector<uint32_t> h(2 * pad32h(top) + 1);
+        copy_out(c, h.data(), dids, h.size() * 4);
         sync(c);
-        if (e) throw Error("invalid MoE router");
-        HIP_OK(hipMemcpyAsync(ids, dids, top * 4, hipMemcpyDeviceToHost, c->s));
-        HIP_OK(hipMemcpyAsync(w, dw, top * 4, hipMemcpyDeviceToHost, c->s));
-        sync(c);
+        if (h.back()) throw Error("invalid MoE router");
+        std::memcpy(ids, h.data(), top * 4);
+        std::memcpy(w, h.data() + pad32h(top), top * 4);
     });
 }
 
@@ -1611,11 +1682,11 @@ int qh_argmax(qh_ctx* c, const float* logits, size_t n, uint32_t* out) {
         int32_t* pk = c->sc.as<int32_t>();
         uint32_t* pi = reinterpret_cast<uint32_t*>(pk + 1024);
         uint32_t* misc = pi + 1024;  // [0] counter, [1] out, [2] err
-        HIP_OK(hipMemsetAsync(misc, 0, 16, c->s));
+        clear_words(c, misc, 16);
         hipLaunchKernelGGL(k_argmax, dim3(grid), dim3(kBlock), 0, c->s, ld, (uint32_t)n, pk, pi, misc, misc + 1, misc + 2);
         HIP_OK(hipGetLastError());
         uint32_t h[3];
-        HIP_OK(hipMemcpyAsync(h, misc, 12, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, h, misc, 12);
         sync(c);
         if (h[2]) throw Error("invalid logits");
         *out = h[1];
@@ -1694,8 +1765,8 @@ int qh_attention(qh_ctx* c, const float* q, const float* k, const float* v, size
         const uint32_t nch = geo.nch;
         const float* qd = upload_x(c, c->sa, q, heads * d);
         c->sb.reserve(klen * 8 + 256);
-        HIP_OK(hipMemcpyAsync(c->sb.p, k, klen * 4, hipMemcpyHostToDevice, c->s));
-        HIP_OK(hipMemcpyAsync(c->sb.as<float>() + klen, v, klen * 4, hipMemcpyHostToDevice, c->s));
+        copy_in(c, c->sb.p, k, klen * 4);
+        copy_in(c, c->sb.as<float>() + klen, v, klen * 4);
         c->stats.uploaded_bytes += klen * 8;
         const size_t part = heads * nch * (d + 2);
         c->sc.reserve((part + heads * d + kvheads + 64) * 4);
@@ -1710,7 +1781,7 @@ int qh_attention(qh_ctx* c, const float* q, const float* k, const float* v, size
         a.counter = cnt;
         a.out = dout;
         launch_attention(a, geo, heads, kvheads, d, c->s);
-        HIP_OK(hipMemcpyAsync(out, dout, heads * d * 4, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, out, dout, heads * d * 4);
         sync(c);
     });
 }
@@ -1753,11 +1824,9 @@ int qh_forward(qh_ctx* c, uint32_t token, float* logits, size_t logits_cap, uint
             reset_model(c);
             throw Error("token outside vocabulary");
         }
-        HIP_OK(hipMemcpyAsync(c->acts.tokens + c->pos, &token, 4, hipMemcpyHostToDevice, c->s));
-        put_state(c, (uint32_t)c->pos, (uint32_t)c->pos + 1);
+        put_state(c, (uint32_t)c->pos, (uint32_t)c->pos + 1, &token);
         launch_step(c);
-        if (logits)
-            HIP_OK(hipMemcpyAsync(logits, c->acts.logits, c->cfg.vocab * 4, hipMemcpyDeviceToHost, c->s));
+        if (logits) copy_out(c, logits, c->acts.logits, c->cfg.vocab * 4);
         DevState st = get_state(c);
         if (st.err) fail_step(c, st.err);
         c->pos += 1;
@@ -1778,16 +1847,13 @@ int qh_generate(qh_ctx* c, const uint32_t* prompt, size_t n_prompt, size_t n_new
         if (c->pos + steps > c->context) throw Error("prompt + max-tokens exceed --ctx");
         for (size_t i = 0; i < n_prompt; i++)
             if (prompt[i] >= c->cfg.vocab) throw Error("token outside vocabulary");
-        HIP_OK(hipMemcpyAsync(c->acts.tokens + c->pos, prompt, n_prompt * 4, hipMemcpyHostToDevice, c->s));
+        copy_in(c, c->acts.tokens + c->pos, prompt, n_prompt * 4);
         put_state(c, (uint32_t)c->pos, (uint32_t)(c->pos + n_prompt));
         for (size_t i = 0; i < steps; i++) launch_step(c);
+        if (n_new) copy_out(c, out_tokens, c->acts.tokens + c->pos + n_prompt, n_new * 4);
+        if (logits_last) copy_out(c, logits_last, c->acts.logits, c->cfg.vocab * 4);
         DevState st = get_state(c);
         if (st.err) fail_step(c, st.err);
-        if (n_new)
-            HIP_OK(hipMemcpyAsync(out_tokens, c->acts.tokens + c->pos + n_prompt, n_new * 4, hipMemcpyDeviceToHost, c->s));
-        if (logits_last)
-            HIP_OK(hipMemcpyAsync(logits_last, c->acts.logits, c->cfg.vocab * 4, hipMemcpyDeviceToHost, c->s));
-        sync(c);
         c->pos += steps;
         c->stats.matvecs += matvecs_per_token(c) * steps;
         c->stats.matvec_ms += now_ms() - t0;
@@ -1830,13 +1896,12 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
         // the prompt through the exact token step, one per token, on the
         // device, as the reference's prompt loop does (src/main.rs:250-256)
         auto run_exact = [&] {
-            HIP_OK(hipMemcpyAsync(c->acts.tokens + c->pos, prompt, n * 4, hipMemcpyHostToDevice, c->s));
+            copy_in(c, c->acts.tokens + c->pos, prompt, n * 4);
             put_state(c, (uint32_t)c->pos, (uint32_t)(c->pos + n));
             for (size_t i = 0; i < n; i++) launch_step(c);
+            if (logits) copy_out(c, logits, c->acts.logits, c->cfg.vocab * 4);
             DevState st = get_state(c);
             if (st.err) fail_step(c, st.err);
-            if (logits) HIP_OK(hipMemcpyAsync(logits, c->acts.logits, c->cfg.vocab * 4, hipMemcpyDeviceToHost, c->s));
-            sync(c);
             if (argmax) *argmax = st.argmax;
             c->pos += n;
             c->stats.matvecs += matvecs_per_token(c) * n;
@@ -1854,7 +1919,7 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
         auto& P = c->pf;
         const ModelDims& d = c->dm;
         const uint32_t p_start = (uint32_t)c->pos;
-        HIP_OK(hipMemcpyAsync(c->acts.tokens + p_start, prompt, n * 4, hipMemcpyHostToDevice, c->s));
+        copy_in(c, c->acts.tokens + p_start, prompt, n * 4);
         // the tail (vocab projection + argmax) runs as the step of the last
         // prompt token: tokens[pos + n] receives the greedy id
         put_state(c, (uint32_t)(p_start + n - 1), (uint32_t)(p_start + n - 1));
@@ -1867,10 +1932,10 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
             for (size_t l = 0; l < c->layers.size(); l++) prefill_layer(c, l, S, p0);
         }
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(c->acts.x, P.X + (size_t)(S - 1) * d.hidden, d.hidden * 4, hipMemcpyDeviceToDevice,
-                              c->s));
+        launch_stage(c, c->acts.x, P.X + (size_t)(S - 1) * d.hidden, d.hidden, d.hidden);
         enqueue_tail(c);
         HIP_OK(hipGetLastError());
+        if (logits) copy_out(c, logits, c->acts.logits, c->cfg.vocab * 4);
         DevState st = get_state(c);
         if (st.err) {
             // the prompt's tokens and positions were checked above, so this is
@@ -1882,8 +1947,6 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
             run_exact();
             return;
         }
-        if (logits) HIP_OK(hipMemcpyAsync(logits, c->acts.logits, c->cfg.vocab * 4, hipMemcpyDeviceToHost, c->s));
-        sync(c);
         if (argmax) *argmax = st.argmax;
         c->pos += n;
         c->stats.matvecs += matvecs_per_token(c) * n;
@@ -1939,7 +2002,7 @@ int qh_layer_forward(qh_ctx* c, size_t layer, float* x, size_t pos, const float*
         if (pos >= c->context) throw Error("context limit " + std::to_string(c->context) + " reached");
         const ModelDims& d = c->dm;
         const LayerW& L = c->layers[layer];
-        HIP_OK(hipMemcpyAsync(c->acts.x, x, d.hidden * 4, hipMemcpyHostToDevice, c->s));
+        copy_in(c, c->acts.x, x, d.hidden * 4);
         if (pos) {
             // time-major host history -> head-major device cache
             const size_t kvd = (size_t)d.kvheads * d.head_dim;
@@ -1964,9 +2027,9 @@ int qh_layer_forward(qh_ctx* c, size_t layer, float* x, size_t pos, const float*
         else
             enqueue_layer(c, layer, false);
         HIP_OK(hipGetLastError());
-        HIP_OK(hipMemcpyAsync(x, c->acts.x, d.hidden * 4, hipMemcpyDeviceToHost, c->s));
-        if (ids) HIP_OK(hipMemcpyAsync(ids, c->acts.ids, d.top * 4, hipMemcpyDeviceToHost, c->s));
-        if (w) HIP_OK(hipMemcpyAsync(w, c->acts.wts, d.top * 4, hipMemcpyDeviceToHost, c->s));
+        copy_out(c, x, c->acts.x, d.hidden * 4);
+        if (ids) copy_out(c, ids, c->acts.ids, d.top * 4);
+        if (w) copy_out(c, w, c->acts.wts, d.top * 4);
         DevState st = get_state(c);
         reset_model(c);
         if (st.err) fail_step(c, st.err);

@@ -30,6 +30,28 @@ __global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t* __restrict__ p, s
     for (size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (size_t)gridDim.x * kBlock) p[i] = v;
 }
 
+// dst[0, n) = src[0, n), dst[n, padded) = 0 (32-bit words): copies between
+// device memory and the engine's pinned host memory, 16 bytes per lane where
+// both sides are aligned.  A kernel in the stream costs a launch (about 3 us of
+// host time); hipMemcpyAsync on a caller's pageable memory 10-20 us a call, and
+// it returns only when the copy is done.
+__global__ __launch_bounds__(kBlock) void k_stage(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src,
+                                                  uint32_t n, uint32_t padded) {
+    const uint32_t i0 = blockIdx.x * kBlock + threadIdx.x, stride = gridDim.x * kBlock;
+    const bool vec = ((reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) & 15) == 0;
+    const uint32_t n4 = vec ? n / 4 : 0;
+    for (uint32_t i = i0; i < n4; i += stride) reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+    for (uint32_t i = 4 * n4 + i0; i < padded; i += stride) dst[i] = i < n ? src[i] : 0u;
+}
+
+// The step state before a call, and (token_at not null) the token it runs.
+__global__ void k_put_state(DevState* st, uint32_t pos, uint32_t n_given, uint32_t* token_at, uint32_t token) {
+    if (threadIdx.x == 0) {
+        *st = DevState{pos, n_given, 0u, 0u, {0u, 0u, 0u, 0u}};
+        if (token_at) *token_at = token;
+    }
+}
+
 // Bit-exact dequantisation of rows [0, rows) (src/quant.rs:81-84).
 __global__ __launch_bounds__(kBlock) void k_dequant(DevMat m, size_t row0, size_t rows, float* __restrict__ out) {
     const size_t total = rows * m.cols;
