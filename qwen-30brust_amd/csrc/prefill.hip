@@ -59,6 +59,34 @@ typedef float f16v __attribute__((ext_vector_type(16)));
 
 template <uint32_t KIND> struct WReg;
 
+// A tile block as WReg::load reads it: the bytes at a lane offset plus a
+// wave-uniform one.  TileBuf (the 128-row tiles): through a buffer resource
+// over the wave's 32 rows, which leaves the per-load address to the scalar
+// unit; 64-bit pointers took a VALU add and two registers each there (Q6_K down
+// 119 -> 109 us at 2,048 tokens: three waves per SIMD instead of two).  TilePtr
+// (tiles of fewer rows): plain pointers; with buffer loads the compiler moved
+// so many of them up that the 32-row gate/up kernels spilled (up to 15 % longer).
+__device__ __forceinline__ uint4 tld16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
+}
+struct TileBuf {
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t at;
+    __device__ __forceinline__ uint4 u4(uint32_t voff, uint32_t soff) const { return tld16(r, voff, at + soff); }
+    __device__ __forceinline__ uint32_t u32(uint32_t voff, uint32_t soff) const {
+        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)(at + soff), 0);
+    }
+    __device__ __forceinline__ uint32_t u16(uint32_t voff, uint32_t soff) const {
+        return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(r, (int)voff, (int)(at + soff), 0);
+    }
+};
+struct TilePtr {
+    const uint8_t* p;
+    __device__ __forceinline__ uint4 u4(uint32_t voff, uint32_t soff) const { return ld16(p + soff + voff); }
+    __device__ __forceinline__ uint32_t u32(uint32_t voff, uint32_t soff) const { return gld<uint32_t>(p + soff + voff); }
+    __device__ __forceinline__ uint32_t u16(uint32_t voff, uint32_t soff) const { return ld_u16(p + soff + voff); }
+};
+
 // Four fp16 values a * (byte i of m) + b, i = 0..3, into v[o .. o+3], from
 // c = b - 1024 a: v_perm_b32 puts byte i under the fp16 exponent of 1024
 // (the half 0x64XX is exactly 1024 + XX), and one v_fma_mix per value
@@ -84,6 +112,52 @@ __device__ __forceinline__ uint32_t and_opaque(uint32_t w, uint32_t mk) {
     return r;
 }
 
+// For the 128-row tiles (gemm_tile_r), the same with one instruction per value
+// (v_fma_mixlo/hi), in assembly: from the expressions above the compiler makes
+// three of four pairs an f32 fma_mix each and a v_cvt_pk, and at 128 rows the
+// dequantisation's VALU instructions, at 4 cycles each, take as long as the
+// products (181 VALU instructions and 32 waits -> 143 and none per gate/up
+// slice).  The halves 1024 + u_i come as (u0, u2) in t0 and (u1, u3) in t1.
+// The closing s_nop belongs to it: a VALU result needs two wait states before
+// an MFMA reads it, which the compiler inserts only behind instructions it
+// sees.  Tiles of fewer rows, whose products follow each dequantisation at
+// once, stay with the compiler's form (this one took them 1-3 % longer).
+__device__ __forceinline__ void halves_mix(h8v& v, int o, uint32_t t0, uint32_t t1, float a, float c) {
+    uint32_t d0, d1;
+    asm("v_fma_mixlo_f16 %0, %2, %4, %5 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixlo_f16 %1, %2, %4, %5 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixhi_f16 %0, %3, %4, %5 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixhi_f16 %1, %3, %4, %5 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+        "s_nop 1"
+        : "=&v"(d0), "=&v"(d1)
+        : "v"(t0), "v"(t1), "v"(a), "v"(c));
+    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+    u4v r = __builtin_bit_cast(u4v, v);
+    r[o / 2] = d0;
+    r[o / 2 + 1] = d1;
+    v = __builtin_bit_cast(h8v, r);
+}
+__device__ __forceinline__ void bytes_mix(h8v& v, int o, uint32_t m, float a, float c) {
+    halves_mix(v, o, __builtin_amdgcn_perm(0x64646464u, m, 0x04020400u),
+               __builtin_amdgcn_perm(0x64646464u, m, 0x04030401u), a, c);
+}
+// A constant the optimiser cannot see, in a scalar (vector) register: as
+// and_opaque, but the and itself may merge with what follows.
+__device__ __forceinline__ uint32_t opaque_s(uint32_t v) {
+    asm("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ uint32_t opaque_v(uint32_t v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// The word of a lane's 16 bytes that holds half H (four values) of k-step S:
+// bytes 8(S%2) + 4H ..
+template <int S, int H> __device__ __forceinline__ uint32_t word4(const uint4& q) {
+    return (S & 1) ? (H ? q.w : q.z) : (H ? q.y : q.x);
+}
+
 template <> struct WReg<Q4_K> {
     uint4 q, hdr;
     // d*sc and the bytes_affine bias of -dmin*m of sub-blocks 2sl (low
@@ -92,9 +166,10 @@ template <> struct WReg<Q4_K> {
     struct Sc { float a0, b0, a1, b1; };
     // from tile block blk (32 rows, one super-block): the lane's row header
     // and quant bytes 32 sl + 16 g .. of its row
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t sl, uint32_t lane) {
-        hdr = ld16(blk + (lane & 31) * 16);
-        q = ld16(blk + 512 + sl * 1024 + lane * 16);
+    template <class T>
+    __device__ __forceinline__ void load(const T& blk, uint32_t sl, uint32_t lane) {
+        hdr = blk.u4((lane & 31) * 16, 0);
+        q = blk.u4(lane * 16, 512 + sl * 1024);
     }
     __device__ __forceinline__ Sc prep(uint32_t sl, uint32_t) const {
         uint32_t scp, mp;
@@ -115,6 +190,14 @@ template <> struct WReg<Q4_K> {
         bytes_affine(v, 4, and_opaque(w1, mk), a, b);
         return v;
     }
+    // half H of it, for the 128-row tiles: a nibble's place in a byte fits the
+    // mantissa of 1024 as it is, so one and-or per two values, no byte permute
+    template <int S, int H>
+    __device__ __forceinline__ void dequant4(h8v& v, const Sc& c, uint32_t) const {
+        const uint32_t w = word4<S, H>(q), mk = opaque_s(S < 2 ? 0x000f000fu : 0x00f000f0u);
+        const uint32_t one = opaque_v(0x64006400u);
+        halves_mix(v, 4 * H, (w & mk) | one, ((w >> 8) & mk) | one, S < 2 ? c.a0 : c.a1, S < 2 ? c.b0 : c.b1);
+    }
 };
 
 template <> struct WReg<Q6_K> {
@@ -127,13 +210,14 @@ template <> struct WReg<Q6_K> {
     // block blk: low-bit bytes 64c + 16g .. and 64c + 32 + 16g .. of the
     // lane's row (columns 16g.. and 32+16g..), their high-bit bytes
     // 32c + 16g .., the slice's 4 scales and d
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t sl, uint32_t lane) {
+    template <class T>
+    __device__ __forceinline__ void load(const T& blk, uint32_t sl, uint32_t lane) {
         const uint32_t c = sl >> 1;
-        l0 = ld16(blk + c * 2048 + lane * 16);
-        l1 = ld16(blk + c * 2048 + 1024 + lane * 16);
-        qh = ld16(blk + 4096 + c * 1024 + lane * 16);
-        sc4 = gld<uint32_t>(blk + 6144 + sl * 128 + (lane & 31) * 4);
-        d = ld_u16(blk + 6656 + (lane & 31) * 2);
+        l0 = blk.u4(lane * 16, c * 2048);
+        l1 = blk.u4(lane * 16, c * 2048 + 1024);
+        qh = blk.u4(lane * 16, 4096 + c * 1024);
+        sc4 = blk.u32((lane & 31) * 4, 6144 + sl * 128);
+        d = blk.u16((lane & 31) * 2, 6656);
     }
     __device__ __forceinline__ Sc prep(uint32_t, uint32_t grp) const {
         const float df = h2f(d);
@@ -158,6 +242,15 @@ template <> struct WReg<Q6_K> {
         bytes_affine(v, 4, vb, a, b);
         return v;
     }
+    // half H of it, for the 128-row tiles
+    template <int S, int H>
+    __device__ __forceinline__ void dequant4(h8v& v, const Sc& c, uint32_t p) const {
+        const uint32_t hs = 2 * (2 * p + (S < 2 ? 0 : 1)), ls = 4 * p;
+        const uint32_t h = word4<S, H>(qh), hi = hs < 4 ? h << (4 - hs) : h >> (hs - 4);
+        const uint32_t w = (hi & opaque_s(0x30303030u)) |
+                           ((word4<S, H>(S < 2 ? l0 : l1) >> ls) & opaque_s(0x0f0f0f0fu));
+        bytes_mix(v, 4 * H, w, S < 2 ? c.a0 : c.a1, S < 2 ? c.b0 : c.b1);
+    }
 };
 
 template <> struct WReg<Q5_K> {
@@ -167,10 +260,11 @@ template <> struct WReg<Q5_K> {
     struct Sc { float a0, b0, a1, b1; uint32_t hs; };
     // from tile block blk: the lane's row header, quant bytes 32 sl + 16 g ..
     // and high-bit bytes 16 g .. of its row
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t sl, uint32_t lane) {
-        hdr = ld16(blk + (lane & 31) * 16);
-        q = ld16(blk + 512 + sl * 1024 + lane * 16);
-        qh = ld16(blk + 4608 + lane * 16);
+    template <class T>
+    __device__ __forceinline__ void load(const T& blk, uint32_t sl, uint32_t lane) {
+        hdr = blk.u4((lane & 31) * 16, 0);
+        q = blk.u4(lane * 16, 512 + sl * 1024);
+        qh = blk.u4(lane * 16, 4608);
     }
     __device__ __forceinline__ Sc prep(uint32_t sl, uint32_t) const {
         uint32_t scp, mp;
@@ -195,6 +289,14 @@ template <> struct WReg<Q5_K> {
         bytes_affine(v, 4, vb, a, b);
         return v;
     }
+    // half H of it, for the 128-row tiles
+    template <int S, int H>
+    __device__ __forceinline__ void dequant4(h8v& v, const Sc& c, uint32_t) const {
+        const uint32_t ls = S < 2 ? 0 : 4, hs = c.hs + (S < 2 ? 0 : 1);
+        const uint32_t h = word4<S, H>(qh), hi = hs < 4 ? h << (4 - hs) : h >> (hs - 4);
+        const uint32_t w = (hi & opaque_s(0x10101010u)) | ((word4<S, H>(q) >> ls) & opaque_s(0x0f0f0f0fu));
+        bytes_mix(v, 4 * H, w, S < 2 ? c.a0 : c.a1, S < 2 ? c.b0 : c.b1);
+    }
 };
 
 // d of blocks 2sl and 2sl+1 (32-column blocks) from the row's eight d
@@ -211,10 +313,11 @@ template <> struct WReg<Q4_0> {
     struct Sc { float a0, b0, a1, b1; uint32_t sh; };
     // from tile block blk: the lane's row's d values and the 16 quant bytes
     // of blocks 2sl and 2sl+1 (both lane groups read the same bytes)
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t sl, uint32_t lane) {
-        dd = ld16(blk + (lane & 31) * 16);
-        q0 = ld16(blk + 512 + sl * 1024 + (lane & 31) * 16);
-        q1 = ld16(blk + 512 + sl * 1024 + 512 + (lane & 31) * 16);
+    template <class T>
+    __device__ __forceinline__ void load(const T& blk, uint32_t sl, uint32_t lane) {
+        dd = blk.u4((lane & 31) * 16, 0);
+        q0 = blk.u4((lane & 31) * 16, 512 + sl * 1024);
+        q1 = blk.u4((lane & 31) * 16, 1024 + sl * 1024);
     }
     __device__ __forceinline__ Sc prep(uint32_t sl, uint32_t grp) const {
         const uint32_t w = d_pair(dd, sl);
@@ -233,6 +336,12 @@ template <> struct WReg<Q4_0> {
         bytes_affine(v, 4, and_opaque(w1 >> c.sh, 0x0f0f0f0fu), a, b);
         return v;
     }
+    // half H of it, for the 128-row tiles
+    template <int S, int H>
+    __device__ __forceinline__ void dequant4(h8v& v, const Sc& c, uint32_t) const {
+        bytes_mix(v, 4 * H, ((word4<S, H>(S < 2 ? q0 : q1) >> c.sh) & opaque_s(0x0f0f0f0fu)), S < 2 ? c.a0 : c.a1,
+                     S < 2 ? c.b0 : c.b1);
+    }
 };
 
 template <> struct WReg<Q8_0> {
@@ -241,10 +350,11 @@ template <> struct WReg<Q8_0> {
     struct Sc { float a0, b0, a1, b1; };
     // from tile block blk: the lane's row's d values and quant bytes 16g ..
     // of blocks 2sl and 2sl+1
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t sl, uint32_t lane) {
-        dd = ld16(blk + (lane & 31) * 16);
-        q0 = ld16(blk + 512 + sl * 2048 + lane * 16);
-        q1 = ld16(blk + 512 + sl * 2048 + 1024 + lane * 16);
+    template <class T>
+    __device__ __forceinline__ void load(const T& blk, uint32_t sl, uint32_t lane) {
+        dd = blk.u4((lane & 31) * 16, 0);
+        q0 = blk.u4(lane * 16, 512 + sl * 2048);
+        q1 = blk.u4(lane * 16, 1536 + sl * 2048);
     }
     __device__ __forceinline__ Sc prep(uint32_t sl, uint32_t) const {
         const uint32_t w = d_pair(dd, sl);
@@ -263,14 +373,20 @@ template <> struct WReg<Q8_0> {
         bytes_affine(v, 4, w1 ^ 0x80808080u, a, b);
         return v;
     }
+    // half H of it, for the 128-row tiles
+    template <int S, int H>
+    __device__ __forceinline__ void dequant4(h8v& v, const Sc& c, uint32_t) const {
+        bytes_mix(v, 4 * H, word4<S, H>(S < 2 ? q0 : q1) ^ 0x80808080u, S < 2 ? c.a0 : c.a1, S < 2 ? c.b0 : c.b1);
+    }
 };
 
 // Weight row of this thread (tile column): wave w, lane l -> 32w + l%32.
 __device__ __forceinline__ uint32_t rtile_row() { return 32 * (threadIdx.x >> 6) + (threadIdx.x & 31); }
-// Tile row of this thread's A load i (i < 4): 32w + 8i + l/8.
-__device__ __forceinline__ uint32_t arow_row(uint32_t i) {
-    return 32 * (threadIdx.x >> 6) + 8 * i + ((threadIdx.x & 63) >> 3);
-}
+// This thread's wave, in a scalar register (and with it what derives from it).
+__device__ __forceinline__ uint32_t wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+// Tile row of this thread's A load i (i < 4): 32i + 8w + l/8, so that the
+// first MB loads of the four waves are row blocks 0 .. MB - 1.
+__device__ __forceinline__ uint32_t arow_row(uint32_t i) { return 32 * i + (threadIdx.x >> 3); }
 
 // Output element acc[.][mb][i] of this lane: tile row / tile column.
 __device__ __forceinline__ uint32_t racc_row(uint32_t mb, uint32_t i) {
@@ -280,95 +396,130 @@ __device__ __forceinline__ uint32_t racc_col() { return rtile_row(); }
 
 constexpr int kRA = 2 * kGM * kGL;  // halfs of LDS: the two A buffers
 
-// acc[nb][mb] += A[m0 .. m0+128) x W_nb[n0 .. n0+128)^T over columns
-// [kbeg, kbeg + K) (kbeg a multiple of 256, K of 64 * STAGES; STAGES even).
-// arows[i]: the A row of tile row arow_row(i) (any valid row past the tile's
-// rows: those outputs are not stored); wblk[nb]: tile block (G, 0) of matrix
-// nb for this wave's row group G = (n0 + 32w) / 32 (likewise clamped).  STAGES register stages
-// of weight loads run ahead; the loads are unconditional (clamped), so each
-// wait covers exactly one stage.  With full false (workgroup-uniform: a tile
-// whose valid rows fit in the first 64) row blocks 2 and 3 are skipped, and
-// acc[.][2..3] stay as they are.
-template <uint32_t KIND, int NB, int STAGES>
-__device__ __forceinline__ void gemm_tile_r(const _Float16* const (&arows)[4], const uint8_t* const (&wblk)[NB],
-                                            uint32_t K, f16v (&acc)[NB][4], _Float16* As, uint32_t kbeg = 0,
-                                            bool full = true) {
-    const uint32_t tid = threadIdx.x, lane = tid & 63, grp = lane >> 5;
-    static_assert(STAGES % 2 == 0, "slice k uses A buffer k % 2 = its stage's parity");
+// acc[nb][mb] += A[m0 .. m0 + 32 MB) x W_nb[n0 .. n0+128)^T over columns
+// [kbeg, kbeg + K) (both multiples of 256), mb < MB.  arows[i]: the A row of
+// tile row arow_row(i) (any valid row past the tile's rows: those outputs are
+// not stored), as a byte offset into A (a chunk's activations are far below 2^32
+// bytes); wblk[nb]: tile block (G, 0) of matrix nb for this wave's row
+// group G = (n0 + 32w) / 32 (likewise clamped, wave-uniform).
+//
+// Bound: the matrix cores (MB NB products of 32 cycles per k-step and wave)
+// against the dequantisation (14-24 VALU instructions of 4 cycles per product
+// column block) and LDS reads of the same k-step, at two waves per SIMD.  So
+// the loop is one software pipeline over k-steps: while a k-step's products
+// run, the next one's B values are dequantised, a quarter of them behind each
+// MB / 2 products, and each A fragment is read again from LDS right behind
+// its last product, which gives the read the rest of the k-step to arrive
+// (single fragment registers: their reuse is in program order).  The last
+// k-step of a slice reads the next slice's first fragments, so its barrier
+// sits in the middle of that k-step, behind half of the products.  The
+// sched_barriers keep the compiler from sorting the k-step back into reads,
+// dequantisation, products.  Against a loop that read, dequantised and
+// multiplied k-step by k-step, with halves_mix, the buffer loads and the tile
+// order of k_pf_group: four layers at 2,048 tokens 2,436 -> 2,346 us, two layers
+// at 1,500 of Q6_K 1,115 -> 1,005, Q5_K_M 1,046 -> 993, Q4_0 984 -> 930, Q8_0
+// 1,011 -> 977, bit for bit the same.  What is left (gate/up at 2,048 tokens: 167
+// us, 39 % matrix-core busy): with every load in the first-level cache it takes
+// 161 us, without the dequantisation 130; the rest is each workgroup's start
+// and SwiGLU and the last of its 2-3 rounds over the chip.
+template <uint32_t KIND, int NB, int MB>
+__device__ __forceinline__ void gemm_tile_r(const _Float16* A, const uint32_t (&arows)[4],
+                                            const uint8_t* const (&wblk)[NB], uint32_t K, f16v (&acc)[NB][4],
+                                            _Float16* As, uint32_t kbeg = 0) {
+    static_assert(MB % 2 == 0, "2 NB groups of MB / 2 products per k-step");
+    const uint32_t lane = threadIdx.x & 63, grp = lane >> 5, ach = threadIdx.x & 7;
     const uint32_t nsl = K / kGK;
-    WReg<KIND> wr[STAGES][NB];
-    uint4 av[2][4];  // A slices k+1 and k+2 in flight while slice k is multiplied
-    auto wload = [&](int st, uint32_t k) {
+    WReg<KIND> wr[2][NB];
+    typename WReg<KIND>::Sc sc[NB];
+    uint4 av[MB];
+    h8v af[MB], bf[2][NB];
+    __amdgpu_buffer_rsrc_t wrs[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; nb++) wrs[nb] = buf_rsrc(wblk[nb], (kbeg + K) / 256 * tile_block_bytes(KIND));
+    const __amdgpu_buffer_rsrc_t ars = buf_rsrc(A, 0xffffffffu);
+    auto wload = [&](auto ST_, uint32_t k) {
         const uint32_t k0 = kbeg + min(k, nsl - 1) * kGK;  // past the end: a harmless reload
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) wr[st][nb].load(wblk[nb] + (size_t)(k0 >> 8) * tile_block_bytes(KIND), (k0 >> 6) & 3, lane);
+        for (int nb = 0; nb < NB; nb++)
+            wr[decltype(ST_)::value][nb].load(TileBuf{wrs[nb], (k0 >> 8) * tile_block_bytes(KIND)}, (k0 >> 6) & 3, lane);
     };
-    // A row r, 16-byte chunks 2i + grp of the slice (lanes l and l+32 read
-    // adjacent chunks of one row)
     // A: load i of a wave covers 8 whole 128-byte slice rows, rows
-    // arow_row(i) (lane l: row 32w + 8i + l/8, 16-byte chunk l%8)
-    const uint32_t ach = lane & 7;
-    auto aload = [&](int j, uint32_t k) {
+    // arow_row(i), 16-byte chunk l%8
+    auto aload = [&](uint32_t k) {
         const uint32_t k0 = kbeg + min(k, nsl - 1) * kGK;
 #pragma unroll
-        for (int i = 0; i < 4; i++) av[j][i] = gld<uint4>(arows[i] + k0 + 8 * ach);
+        for (int i = 0; i < MB; i++) av[i] = tld16(ars, arows[i] + 16 * ach, 2 * k0);
     };
-    // A slice held in av[j] to LDS buffer j (slice k sits in buffer k % 2)
-    auto astore = [&](int j) {
+    // slice k sits in LDS buffer k % 2
+    auto astore = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            *reinterpret_cast<uint4*>(As + j * kGM * kGL + arow_row(i) * kGL + 8 * ach) = av[j][i];
+        for (int i = 0; i < MB; i++)
+            *reinterpret_cast<uint4*>(As + buf * kGM * kGL + arow_row(i) * kGL + 8 * ach) = av[i];
     };
-#pragma unroll
-    for (int st = 0; st < STAGES; st++) wload(st, st);
-    aload(0, 0);
+    const _Float16* const afp = As + (lane & 31) * kGL + 16 * grp;
+    auto aread = [&](int buf, int S, int mb) {
+        af[mb] = *reinterpret_cast<const h8v*>(afp + buf * kGM * kGL + 32 * mb * kGL + 32 * (S >> 1) + 8 * (S & 1));
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    wload(I0{}, 0);
+    aload(0);
+    wload(I1{}, 1);
     astore(0);
-    aload(1, 1);
-    aload(0, 2);
+    aload(1);
     __syncthreads();
-    for (uint32_t k0 = 0; k0 < nsl; k0 += STAGES) {
 #pragma unroll
-        for (int st = 0; st < STAGES; st++) {
-            const uint32_t k = k0 + st;
-            const uint32_t sl = ((kbeg >> 6) + k) & 3, p = sl & 1;
-            const _Float16* Ab = As + (k & 1) * kGM * kGL;
-            typename WReg<KIND>::Sc sc[NB];
+    for (int mb = 0; mb < MB; mb++) aread(0, 0, mb);
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) sc[nb] = wr[st][nb].prep(sl, grp);
-            auto kstep = [&](auto S_) {
-                constexpr int S = decltype(S_)::value;
-                const uint32_t col = 32 * (S >> 1) + 16 * grp + 8 * (S & 1);
-                h8v af[4], bf[NB];
+    for (int nb = 0; nb < NB; nb++) {
+        sc[nb] = wr[0][nb].prep(0, grp);
+        bf[0][nb] = wr[0][nb].template dequant<0>(sc[nb], 0);
+    }
+    // k-step S of slice k, the slice SL of its super-block
+    auto kstep = [&](auto SL_, auto S_, uint32_t k) {
+        constexpr int SL = decltype(SL_)::value, S = decltype(S_)::value, ST = SL & 1;
+        constexpr int SN = (S + 1) & 3, SLN = S == 3 ? (SL + 1) & 3 : SL, STN = SLN & 1;  // the next k-step
+        auto group = [&](auto G_) {
+            constexpr int G = decltype(G_)::value;
 #pragma unroll
-                for (int mb = 0; mb < 2; mb++)
-                    af[mb] = *reinterpret_cast<const h8v*>(Ab + (32 * mb + (lane & 31)) * kGL + col);
+            for (int j = G * MB / 2; j < (G + 1) * MB / 2; j++) {
+                const int mb = j / NB, nb = j % NB;
+                acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf[S & 1][nb], acc[nb][mb], 0, 0, 0);
+                if (nb == NB - 1 && (S < 3 || mb >= MB / 2)) aread(STN, SN, mb);
+            }
+            constexpr int nb = G / 2, H = G & 1;
+            if constexpr (S == 3 && H == 0) sc[nb] = wr[STN][nb].prep(SLN, grp);
+            wr[STN][nb].template dequant4<SN, H>(bf[1 - (S & 1)][nb], sc[nb], SLN & 1);
+            if constexpr (S == 1 && G == 0) {
+                astore(1 - ST);  // slice k + 1; the readers of k - 1 passed its barrier
+                aload(k + 2);
+            }
+            if constexpr (S == 3 && G == 0) wload(std::integral_constant<int, ST>{}, k + 2);
+            if constexpr (S == 3 && G == NB - 1) {
+                __syncthreads();  // slice k + 1 is stored, and k's reads are done
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++) bf[nb] = wr[st][nb].template dequant<S>(sc[nb], p);
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                    for (int mb = 0; mb < 2; mb++)
-                        acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf[nb], acc[nb][mb], 0, 0, 0);
-                if (full) {
-#pragma unroll
-                    for (int mb = 2; mb < 4; mb++)
-                        af[mb] = *reinterpret_cast<const h8v*>(Ab + (32 * mb + (lane & 31)) * kGL + col);
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                        for (int mb = 2; mb < 4; mb++)
-                            acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mb], bf[nb], acc[nb][mb], 0, 0, 0);
-                }
-            };
-            kstep(std::integral_constant<int, 0>{});
-            kstep(std::integral_constant<int, 1>{});
-            kstep(std::integral_constant<int, 2>{});
-            kstep(std::integral_constant<int, 3>{});
-            wload(st, k + STAGES);
-            astore((st + 1) & 1);  // slice k + 1
-            aload((st + 1) & 1, k + 3);
-            __syncthreads();
+                for (int mb = 0; mb < MB / 2; mb++) aread(STN, SN, mb);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        group(I0{});
+        group(I1{});
+        if constexpr (NB == 2) {
+            group(std::integral_constant<int, 2>{});
+            group(std::integral_constant<int, 3>{});
         }
+    };
+    auto slice = [&](auto SL_, uint32_t k) {
+        kstep(SL_, I0{}, k);
+        kstep(SL_, I1{}, k);
+        kstep(SL_, std::integral_constant<int, 2>{}, k);
+        kstep(SL_, std::integral_constant<int, 3>{}, k);
+    };
+    for (uint32_t k = 0; k < nsl; k += 4) {
+        slice(I0{}, k);
+        slice(I1{}, k + 1);
+        slice(std::integral_constant<int, 2>{}, k + 2);
+        slice(std::integral_constant<int, 3>{}, k + 3);
     }
 }
 
@@ -400,7 +551,7 @@ __device__ __forceinline__ void gemm_skinny(const _Float16* const (&arows)[4], c
         for (int nb = 0; nb < NB; nb++)
 #pragma unroll
             for (int sl = 0; sl < WS; sl++)
-                wr[decltype(B_)::value][nb][sl].load(wblk[nb] + o, WS * decltype(G_)::value + sl, lane);
+                wr[decltype(B_)::value][nb][sl].load(TilePtr{wblk[nb] + o}, WS * decltype(G_)::value + sl, lane);
     };
     auto aload = [&](uint32_t j) {  // staged part j: columns 256 sb0 + 64 KS j ..
         const uint32_t k0 = 256 * sb0 + 64 * KS * min(j, MB * nsb - 1);
@@ -486,14 +637,11 @@ __global__ __launch_bounds__(kGT, 2) void k_gemm_gateup(const _Float16* Xn, uint
     if (ty >= *G.ntile) return;
     const uint32_t e = G.te[ty], mt0 = G.tm[ty];
     const uint32_t base = G.goff[e], rows = G.goff[e + 1] - base;
-    const uint32_t n0 = tx * kGN, r = rtile_row(), ff = Wg.rows;
-    const _Float16* arows[4];
+    const uint32_t n0 = tx * kGN, ff = Wg.rows;
+    uint32_t arows[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t ra = mt0 + arow_row(i);
-        arows[i] = Xn + (size_t)(ra < rows ? G.tok[base + ra] : 0u) * H;
-    }
-    const size_t gofs = (size_t)min((n0 >> 5) + (threadIdx.x >> 6), ff / 32 - 1) * tile_group_bytes(KIND, Wg.cols);
+    for (int i = 0; i < 4; i++) arows[i] = G.tok[base + min(mt0 + arow_row(i), rows - 1)] * H * 2;
+    const size_t gofs = (size_t)min((n0 >> 5) + wave_id(), ff / 32 - 1) * tile_group_bytes(KIND, Wg.cols);
     const uint8_t* const wblk[2] = {Wg.wt + e * Wg.expert_stride + gofs, Wu.wt + e * Wu.expert_stride + gofs};
     f16v acc[2][4];
 #pragma unroll
@@ -502,7 +650,8 @@ __global__ __launch_bounds__(kGT, 2) void k_gemm_gateup(const _Float16* Xn, uint
         for (int mb = 0; mb < 4; mb++) acc[nb][mb] = f16v{};
     // a tile of at most 64 valid rows (an expert's remainder past its full
     // tiles) multiplies two row blocks, not four
-    gemm_tile_r<KIND, 2, 2>(arows, wblk, Wg.cols, acc, smem, 0, rows - mt0 > 64);
+    if (rows - mt0 > 64) gemm_tile_r<KIND, 2, 4>(Xn, arows, wblk, Wg.cols, acc, smem);
+    else gemm_tile_r<KIND, 2, 2>(Xn, arows, wblk, Wg.cols, acc, smem);
     const uint32_t n = n0 + racc_col();
     bool bad = false;
 #pragma unroll
@@ -529,19 +678,20 @@ __global__ __launch_bounds__(kGT, 2) void k_gemm_down(const _Float16* Hs, Expert
     if (ty >= *G.ntile) return;
     const uint32_t e = G.te[ty], mt0 = G.tm[ty];
     const uint32_t base = G.goff[e], rows = G.goff[e + 1] - base;
-    const uint32_t n0 = tx * kGN, r = rtile_row(), ff = Wd.cols, N = Wd.rows;
+    const uint32_t n0 = tx * kGN, ff = Wd.cols, N = Wd.rows;
     // visible to the epilogue through the GEMM's barriers
     if (threadIdx.x < kGM) dsts[threadIdx.x] = G.asg[base + min(mt0 + threadIdx.x, rows - 1)];
-    const _Float16* arows[4];
+    uint32_t arows[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) arows[i] = Hs + (size_t)(base + min(mt0 + arow_row(i), rows - 1)) * ff;
+    for (int i = 0; i < 4; i++) arows[i] = (base + min(mt0 + arow_row(i), rows - 1)) * ff * 2;
     const uint8_t* const wblk[1] = {
         Wd.wt + e * Wd.expert_stride +
-        (size_t)min((n0 >> 5) + (threadIdx.x >> 6), N / 32 - 1) * tile_group_bytes(KIND, Wd.cols)};
+        (size_t)min((n0 >> 5) + wave_id(), N / 32 - 1) * tile_group_bytes(KIND, Wd.cols)};
     f16v acc[1][4];
 #pragma unroll
     for (int mb = 0; mb < 4; mb++) acc[0][mb] = f16v{};
-    gemm_tile_r<KIND, 1, 2>(arows, wblk, ff, acc, smem, 0, rows - mt0 > 64);  // as in k_gemm_gateup
+    if (rows - mt0 > 64) gemm_tile_r<KIND, 1, 4>(Hs, arows, wblk, ff, acc, smem);  // as in k_gemm_gateup
+    else gemm_tile_r<KIND, 1, 2>(Hs, arows, wblk, ff, acc, smem);
     const uint32_t n = n0 + racc_col();
 #pragma unroll
     for (int mb = 0; mb < 4; mb++)
@@ -639,16 +789,16 @@ template <uint32_t KIND>
 __device__ __forceinline__ void dense_body(const _Float16* X16, uint32_t S, const DevMat& W, uint32_t m0,
                                            uint32_t n0, uint32_t kbeg, uint32_t K, float* C, uint32_t ldc,
                                            uint32_t cofs, _Float16* smem) {
-    const uint32_t r = rtile_row(), N = W.rows, ld = W.cols;
-    const _Float16* arows[4];
+    const uint32_t N = W.rows, ld = W.cols;
+    uint32_t arows[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) arows[i] = X16 + (size_t)min(m0 + arow_row(i), S - 1) * ld;
+    for (int i = 0; i < 4; i++) arows[i] = min(m0 + arow_row(i), S - 1) * ld * 2;
     const uint8_t* const wblk[1] = {
-        W.wt + (size_t)min((n0 >> 5) + (threadIdx.x >> 6), N / 32 - 1) * tile_group_bytes(KIND, W.cols)};
+        W.wt + (size_t)min((n0 >> 5) + wave_id(), N / 32 - 1) * tile_group_bytes(KIND, W.cols)};
     f16v acc[1][4];
 #pragma unroll
     for (int mb = 0; mb < 4; mb++) acc[0][mb] = f16v{};
-    gemm_tile_r<KIND, 1, 2>(arows, wblk, K, acc, smem, kbeg);
+    gemm_tile_r<KIND, 1, 4>(X16, arows, wblk, K, acc, smem, kbeg);
     const uint32_t n = n0 + racc_col();
 #pragma unroll
     for (int mb = 0; mb < 4; mb++)
@@ -670,7 +820,7 @@ __device__ __forceinline__ uint32_t xcd_unit(uint32_t units) {
     return (blockIdx.x >> 3) < per ? min(u, units) : units;
 }
 
-// Three workgroups per CU (168 VGPRs, 4 of them spilled): the q|k|v grid of
+// Three workgroups per CU (163 VGPRs): the q|k|v grid of
 // 16 x 40 tiles at 2,048 tokens then runs in one round of 768 workgroup slots
 // rather than 1.25 rounds of 512.
 __global__ __launch_bounds__(kGT, 3) void k_gemm_dense(const _Float16* X16, uint32_t S, DenseSegs G, float* C,
@@ -1162,15 +1312,22 @@ __global__ __launch_bounds__(kBlock) void k_pf_topk(const float* LR, uint32_t S,
 // Groups the S*top (token, slot) assignments by expert (one workgroup):
 // goff = exclusive prefix of the per-expert counts, tok/asg = the
 // assignments sorted by expert (order within an expert is arbitrary), and
-// the list of gm-row GEMM tiles (te, tm).  Up to 16,384 assignments are
+// the list of gm-row GEMM tiles (te, tm): 128-row tiles with the experts' full
+// tiles first, then the remainders over 64 rows, then the short ones, so that
+// the launch ends on its shortest workgroups (its 1,100-1,400 take 2-3 rounds
+// of the chip: gate/up at 2,048 tokens 175 -> 167 us); 32- and 64-row tiles, which
+// the weights bound, in expert order, so that an expert's tiles run together and
+// share its weights (sorted, 64-row tiles took 2 % longer).  Up to 16,384 assignments are
 // placed in LDS first and stored in order (coalesced: stored straight to
 // their sorted positions, every store instruction of a wave touched up to 64
 // cache lines).
 __global__ __launch_bounds__(1024) void k_pf_group(const uint32_t* ids, uint32_t n, uint32_t top, uint32_t E,
                                                    uint32_t gm, uint32_t* goff, uint32_t* tok, uint32_t* asg,
                                                    uint32_t* te, uint32_t* tm, uint32_t* ntile) {
-    __shared__ uint32_t cnt[256], cur[256], tb[256];  // E <= 255
+    __shared__ uint32_t cnt[256], cur[256], tb[256], rb[256];  // E <= 255
     __shared__ uint32_t srt[16384], ntot;              // sorted assignments, their count
+    const bool sorted = gm == kGM;
+    const uint32_t lg = 31 - __clz(gm);  // gm is a power of two
     for (uint32_t e = threadIdx.x; e < 256; e += 1024) cnt[e] = 0;
     // this thread's assignments a = threadIdx.x + 1024 i, all loaded before
     // any is used (one memory round trip instead of one per assignment)
@@ -1190,14 +1347,17 @@ __global__ __launch_bounds__(1024) void k_pf_group(const uint32_t* ids, uint32_t
         if (ids[a] < E) atomicAdd(&cnt[ids[a]], 1u);
     __syncthreads();
     if (threadIdx.x < 64) {
-        // wave 0: exclusive prefix sums of the counts and of the tile counts,
-        // lane l holding experts 4l .. 4l + 3
+        // wave 0: exclusive prefix sums of the counts and of the tile counts
+        // (full tiles, or all of them in expert order: 16 bits; remainder tiles
+        // over, and up to, half a tile: 8 bits each, E <= 255), lane l holding
+        // experts 4l .. 4l + 3
         const uint32_t lane = threadIdx.x;
         uint32_t c4[4], t4[4], cs = 0, ts = 0;
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) {
             c4[k] = cnt[4 * lane + k];  // zero past E
-            t4[k] = (c4[k] + gm - 1) / gm;
+            const uint32_t r = sorted ? c4[k] & (gm - 1) : 0u;
+            t4[k] = ((c4[k] + (sorted ? 0 : gm - 1)) >> lg) + (r == 0 ? 0u : 2 * r > gm ? 1u << 16 : 1u << 24);
             cs += c4[k];
             ts += t4[k];
         }
@@ -1211,25 +1371,28 @@ __global__ __launch_bounds__(1024) void k_pf_group(const uint32_t* ids, uint32_t
             }
         }
         uint32_t off = ci - cs, toff = ti - ts;
+        const uint32_t all = __shfl(ti, 63, 64), nf = all & 0xffffu, nbig = all >> 16 & 0xffu;
 #pragma unroll
         for (uint32_t k = 0; k < 4; k++) {
             const uint32_t e = 4 * lane + k;
             if (e <= E) goff[e] = off;  // goff[E] = total
             cur[e] = off;
-            tb[e] = toff;
+            tb[e] = toff & 0xffffu;
+            rb[e] = nf + (t4[k] >> 24 ? nbig + (toff >> 24) : toff >> 16 & 0xffu);
             off += c4[k];
             toff += t4[k];
         }
         if (lane == 63) {
-            *ntile = ti;
+            *ntile = nf + nbig + (all >> 24);
             ntot = ci;
         }
     }
     __syncthreads();
     for (uint32_t e = threadIdx.x; e < E; e += 1024)
         for (uint32_t m = 0, t = tb[e]; m < cnt[e]; m += gm, t++) {
-            te[t] = e;
-            tm[t] = m;
+            const uint32_t i = sorted && m + gm > cnt[e] ? rb[e] : t;
+            te[i] = e;
+            tm[i] = m;
         }
     const bool staged = n <= 1024 * kPer;  // workgroup-uniform
 #pragma unroll
