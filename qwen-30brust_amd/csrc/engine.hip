@@ -531,7 +531,7 @@ void alloc_acts(qh_ctx* c) {
     size_t total = 0;
     for (auto& p : parts) total += (p.first + 255) / 256 * 256;
     c->acts_buf.alloc(total);
-    HIP_OK(hipMemset(c->acts_buf.p, 0, total));
+    HIP_OK(hipMemsetAsync(c->acts_buf.p, 0, total, c->s));
     size_t off = 0;
     for (auto& p : parts) {
         *p.second = c->acts_buf.as<uint8_t>() + off;
@@ -539,7 +539,7 @@ void alloc_acts(qh_ctx* c) {
     }
     const size_t kv_layer = (size_t)d.kvheads * c->context * d.head_dim;
     c->kv.alloc(kv_layer * 2 * 4 * c->cfg.layers);
-    HIP_OK(hipMemset(c->kv.p, 0, c->kv.n));
+    HIP_OK(hipMemsetAsync(c->kv.p, 0, c->kv.n, c->s));
     build_rope(c);
     a.rope = c->rope_buf.as<const float2>();
 }
@@ -794,7 +794,7 @@ void setup_persist(qh_ctx* c) {
     for (const Region& r : regions) total += up256(r.words * 8);
     c->sync_buf.alloc(total);
     c->sync_bytes = total;
-    HIP_OK(hipMemset(c->sync_buf.p, 0, total));
+    HIP_OK(hipMemsetAsync(c->sync_buf.p, 0, total, c->s));
     uint8_t* q = c->sync_buf.as<uint8_t>();
     A.abort_flag = reinterpret_cast<uint32_t*>(q);
     q += 256;
@@ -1115,7 +1115,9 @@ void prefill_alloc(qh_ctx* c, uint32_t cap) {
     uint64_t total = 0;
     for (const R& r : regs) total += up(r.bytes);
     P.buf.alloc(total);
-    HIP_OK(hipMemset(P.buf.p, 0, total));
+    // in the context's stream, as every clear here: hipMemset runs in the null
+    // stream, which that one does not wait for, and returns before it is done
+    HIP_OK(hipMemsetAsync(P.buf.p, 0, total, c->s));
     uint8_t* q = P.buf.as<uint8_t>();
     for (const R& r : regs) {
         *r.dst = q;
