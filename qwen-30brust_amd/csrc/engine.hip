@@ -1916,6 +1916,9 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
         prefill_tiles(c);
         size_t chunk = kPrefillChunk;
         if (const char* e = std::getenv("QH_PREFILL_CHUNK")) chunk = std::max<long>(1, std::atol(e));
+        // the GEMMs address a chunk's fp16 activations with 32-bit byte offsets
+        const uint64_t widest = std::max<uint64_t>({c->dm.hidden, c->dm.heads * 128ull, (uint64_t)c->dm.top * c->dm.ff});
+        chunk = std::min<size_t>(chunk, std::max<size_t>(1, 0xffffffffull / (2 * widest)));
         const uint32_t cap = (uint32_t)std::min<size_t>({n, chunk, kPrefillChunk, c->context});
         prefill_alloc(c, cap);
         auto& P = c->pf;
