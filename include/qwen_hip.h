@@ -143,15 +143,21 @@ int qh_attention(qh_ctx *ctx, const float *q, const float *k, const float *v, si
  * capture, tight serving loops, harnesses that forbid hipMalloc).  q, k, v
  * and out are device pointers in qh_attention's layouts; the kernel's chunk
  * partials and counters live in fixed 1 MiB device areas of the library
- * (eight per GPU, one per calling stream).  Both entry points cap the key chunks per KV head at what
- * the array holds (a chunk then takes several key tiles), so any history
+ * (eight per GPU).  Both entry points cap the key chunks per KV head at what
+ * an area holds (a chunk then takes several key tiles), so any history
  * length runs; a shape one chunk of whose partials alone exceeds it
  * (heads x (head_dim + 2) floats > 1 MiB) is refused with an error.  stream NULL:
  * the context's stream, and the call returns when out is written; otherwise
  * the work is enqueued on that HIP stream and the call returns at once.
- * Calls on up to eight streams of a GPU may overlap; with more, the stream
- * that called least recently gives up its area, and calls of the two streams
- * that overlap race. */
+ * Calls may overlap, from any streams and host threads (a context's own calls
+ * come from one thread), and a captured call's graph may be replayed on any
+ * stream beside them.  A call takes an area that no call under way on another
+ * stream uses; where there is none, and under graph capture, the attention
+ * runs without scratch, with the same bits for head_dim 64 or 128, at most
+ * eight query heads per KV head and q, k and v aligned to 16 bytes, else with
+ * its sums in another order.  It is slower then for long histories (3,581
+ * keys, 32 / 4 heads of 128: 70 us, 8 with an area).  A stream is destroyed
+ * only when its calls have ended. */
 int qh_attention_noalloc(qh_ctx *ctx, const float *q, const float *k, const float *v, size_t klen,
                          size_t heads, size_t kvheads, size_t d, float *out, void *stream);
 

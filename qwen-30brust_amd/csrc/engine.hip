@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -38,6 +39,9 @@ __global__ void k_argmax(const float*, uint32_t, int32_t*, uint32_t*, uint32_t*,
 __global__ void k_attention_api(AttnArgs, uint32_t);
 template <int D> __global__ void k_attention_tile(AttnArgs, uint32_t);
 template <int D> __global__ void k_attention_merge(AttnArgs, uint32_t);
+template <int D> __global__ void k_attention_direct(AttnArgs, uint32_t);
+template <int E> __global__ void k_attention_any(AttnArgs, uint32_t);
+__global__ void k_attention_wide(AttnArgs, uint32_t);
 // Token-step kernels (step.hip).
 // Template argument C: held chunk slots per lane (tile_slots), 0 = general.
 template <int C> __global__ void k_qkv(LayerW, DevMat, Acts, ModelDims, int);
@@ -180,56 +184,96 @@ uint64_t groups_host(uint64_t rows, uint64_t cols, int R) {
 // Device memory of qh_attention_noalloc: the chunk partials
 // [heads][chunks][d+2] and the last-arrival counters [kvheads] of the
 // attention kernels, at most kNoAllocScratchBytes per call.  Every GPU the
-// library runs on holds kNoAllocSlots such areas for the life of the process,
-// one per stream that calls it, so that calls on different streams do not
-// share one (calls on one stream follow each other).  With more streams than
-// areas, the least recently used area goes to the new stream.  Host code uses
-// only the per-device address that hipGetSymbolAddress returns (the array's
-// name is a host-side stand-in, not a device address).
+// library runs on holds kNoAllocAreas such areas for the life of the process,
+// one per stream that calls it (per host thread for hipStreamPerThread, one
+// handle for a stream per thread): calls of one stream follow each other.  A
+// stream without an area gets one that no call has used, or the least recently
+// used one whose calls have all ended: each workgroup that has read its
+// partials counts in `scratch_done`, and the host compares the count with the
+// calls' total.  It does so only for such a stream, because an event behind
+// every call, the other way to know, took 2.3 us of the 8.1 us that a call
+// over 3,581 keys takes (10.4).  A call waits for no other call: where every
+// area is in use, and under graph capture (a graph may be launched any number
+// of times, on any stream, beside any call), the attention runs without
+// scratch (launch_attention_direct).  Area and kernels are taken under the
+// lock: two host threads that use one stream must not interleave their
+// kernels.  Host code uses only the per-device addresses that
+// hipGetSymbolAddress returns (the arrays' names are host-side stand-ins, not
+// device addresses).
 namespace {
 constexpr size_t kNoAllocScratchBytes = 1u << 20;
-constexpr int kNoAllocSlots = 8;
+constexpr int kNoAllocAreas = 8;
 constexpr int kNoAllocMaxDevices = 64;
-struct ScratchSlots {
+struct ScratchAreas {
+    std::mutex mu;
     uint8_t* base = nullptr;
-    hipStream_t stream[kNoAllocSlots] = {};
-    uint64_t used[kNoAllocSlots] = {};  // time of the slot's last call, 0 = never
+    unsigned long long* done = nullptr;  // device: merging workgroups that have ended, per area
+    unsigned long long* seen = nullptr;  // pinned: `done` as last copied
+    hipStream_t probe = nullptr;         // of that copy
+    struct Area {
+        hipStream_t stream = nullptr;
+        uint64_t thread = 0;             // hipStreamPerThread: whose
+        uint64_t used = 0;               // time of its last call, 0 = never
+        unsigned long long launched = 0; // merging workgroups of its calls
+    } area[kNoAllocAreas];
     uint64_t calls = 0;
 };
-std::mutex g_scratch_mu;
-std::array<ScratchSlots, kNoAllocMaxDevices> g_scratch;
-}  // namespace
-static __device__ __align__(256) uint8_t scratch[kNoAllocSlots * kNoAllocScratchBytes];
+std::array<ScratchAreas, kNoAllocMaxDevices> g_scratch;
 
-// Resolves this device's copy of `scratch` once per device (called by
-// qh_create with the device current).
+// A number of the calling host thread's own, never another one's.
+uint64_t thread_serial() {
+    static std::atomic<uint64_t> next{1};
+    thread_local const uint64_t mine = next++;
+    return mine;
+}
+}  // namespace
+static __device__ __align__(256) uint8_t scratch[kNoAllocAreas * kNoAllocScratchBytes];
+static __device__ unsigned long long scratch_done[kNoAllocAreas];
+
+// Resolves this device's copies of `scratch` and `scratch_done`, once per
+// device (called by qh_create with the device current).
 static void noalloc_init(int device) {
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
     if (device < 0 || device >= kNoAllocMaxDevices) throw Error("device index beyond the scratch table");
-    if (g_scratch[device].base) return;
-    void* p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-    if (e != hipSuccess || p == nullptr)
-        throw Error(std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
-    g_scratch[device].base = static_cast<uint8_t*>(p);
+    ScratchAreas& S = g_scratch[device];
+    std::lock_guard<std::mutex> lock(S.mu);
+    if (S.base) return;
+    auto address = [](const void* symbol) {
+        void* p = nullptr;
+        const hipError_t e = hipGetSymbolAddress(&p, symbol);
+        if (e != hipSuccess || p == nullptr)
+            throw Error(std::string("hipGetSymbolAddress(scratch): ") + hipGetErrorString(e));
+        return p;
+    };
+    S.done = static_cast<unsigned long long*>(address(HIP_SYMBOL(scratch_done)));
+    if (!S.seen) HIP_OK(hipHostMalloc((void**)&S.seen, sizeof(scratch_done)));
+    if (!S.probe) HIP_OK(hipStreamCreateWithFlags(&S.probe, hipStreamNonBlocking));
+    S.base = static_cast<uint8_t*>(address(HIP_SYMBOL(scratch)));
 }
 
-// The scratch area of calls on stream s.
-static uint8_t* noalloc_scratch(int device, hipStream_t s) {
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    ScratchSlots& S = g_scratch[device];
-    if (!S.base) throw Error("no-allocation scratch is not set up on this device");
-    int slot = 0;
-    for (int i = 0; i < kNoAllocSlots; i++) {
-        if (S.used[i] && S.stream[i] == s) {
-            slot = i;
-            break;
-        }
-        if (S.used[i] < S.used[slot]) slot = i;
+// The area for a call on stream s, or null where other streams' calls use all
+// of them (or where that cannot be found out: another thread's capture may
+// forbid the copy).  The caller holds the lock.
+static ScratchAreas::Area* noalloc_area(ScratchAreas& S, hipStream_t s) {
+    const uint64_t thread = s == hipStreamPerThread ? thread_serial() : 0;
+    ScratchAreas::Area* mine = nullptr;
+    for (auto& A : S.area) {
+        if (A.used && A.stream == s && A.thread == thread) return &A;
+        if (!A.used && !mine) mine = &A;
     }
-    S.stream[slot] = s;
-    S.used[slot] = ++S.calls;
-    return S.base + slot * kNoAllocScratchBytes;
+    if (!mine) {
+        if (hipMemcpyAsync(S.seen, S.done, sizeof(scratch_done), hipMemcpyDeviceToHost, S.probe) != hipSuccess ||
+            hipStreamSynchronize(S.probe) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        for (int i = 0; i < kNoAllocAreas; i++)
+            if (S.seen[i] == S.area[i].launched && (!mine || S.area[i].used < mine->used)) mine = &S.area[i];
+    }
+    if (mine) {
+        mine->stream = s;
+        mine->thread = thread;
+    }
+    return mine;
 }
 
 struct qh_ctx {
@@ -1717,7 +1761,8 @@ AttnGeo attn_geometry(size_t klen, size_t heads, size_t kvheads, size_t d) {
     // at most kAttnApiMaxChunks chunks per KV head, fewer when one chunk's
     // partials of every head would not fit the no-allocation scratch that
     // many times: a chunk then takes several tiles (both entry points use
-    // this geometry, so they give the same bits)
+    // this geometry, so they give the same bits where they run the same
+    // kernels: q, k and v aligned to 16 bytes, as qh_attention's own are)
     const size_t tiles = (g.T + g.tc - 1) / g.tc, per_chunk = heads * (d + 2) * 4;
     const size_t fit = (kNoAllocScratchBytes - 4096) / per_chunk;
     const size_t cap = std::max<size_t>(1, std::min<size_t>(kAttnApiMaxChunks, fit));
@@ -1728,11 +1773,8 @@ AttnGeo attn_geometry(size_t klen, size_t heads, size_t kvheads, size_t d) {
     return g;
 }
 
-// Launches the attention of `a` (its q, k, v, part, counter and out set): the
-// register-tiled kernels where they apply, else the general one, whose
-// arrival counters are cleared first (by a fill kernel: no memset node in a
-// captured graph).
-static void launch_attention(AttnArgs a, const AttnGeo& geo, size_t heads, size_t kvheads, size_t d, hipStream_t s) {
+// Fills in the shape of `a`; true where the register-tiled kernels apply.
+static bool attention_shape(AttnArgs& a, const AttnGeo& geo, size_t heads, size_t kvheads, size_t d) {
     a.sh = d;
     a.st = kvheads * d;
     a.heads = (uint32_t)heads;
@@ -1742,22 +1784,53 @@ static void launch_attention(AttnArgs a, const AttnGeo& geo, size_t heads, size_
     a.max_chunks = geo.nch;
     a.span = geo.span;
     a.err = nullptr;
-    const uint32_t T = (uint32_t)geo.T;
     const bool aligned = ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) % 16 == 0;
+    return aligned && (d == 128 || d == 64) && heads / kvheads <= 8;
+}
+
+// Launches the attention of `a` (its q, k, v, part, counter, done and out
+// set): the register-tiled kernels where they apply, else the general one,
+// whose arrival counters are cleared first.  Returns the number of
+// workgroups that count in *a.done; the caller looks at hipGetLastError.
+static uint32_t launch_attention(AttnArgs a, const AttnGeo& geo, size_t heads, size_t kvheads, size_t d,
+                                 hipStream_t s) {
+    const bool tiled = attention_shape(a, geo, heads, kvheads, d);
+    const uint32_t T = (uint32_t)geo.T;
     const dim3 grid((uint32_t)kvheads, geo.nch);
-    if (aligned && (d == 128 || d == 64) && heads / kvheads <= 8) {
-        if (d == 128) {
-            hipLaunchKernelGGL(k_attention_tile<128>, grid, dim3(kBlock), 0, s, a, T);
-            hipLaunchKernelGGL(k_attention_merge<128>, dim3(a.heads), dim3(kBlock), 0, s, a, geo.nch);
-        } else {
-            hipLaunchKernelGGL(k_attention_tile<64>, grid, dim3(kBlock), 0, s, a, T);
-            hipLaunchKernelGGL(k_attention_merge<64>, dim3(a.heads), dim3(kBlock), 0, s, a, geo.nch);
-        }
-    } else {
+    if (!tiled) {
         hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, s, a.counter, kvheads, 0u);
         hipLaunchKernelGGL(k_attention_api, grid, dim3(kBlock), geo.lds, s, a, T);
+        return a.kvheads;
     }
-    HIP_OK(hipGetLastError());
+    if (d == 128) {
+        hipLaunchKernelGGL(k_attention_tile<128>, grid, dim3(kBlock), 0, s, a, T);
+        hipLaunchKernelGGL(k_attention_merge<128>, dim3(a.heads), dim3(kBlock), 0, s, a, geo.nch);
+    } else {
+        hipLaunchKernelGGL(k_attention_tile<64>, grid, dim3(kBlock), 0, s, a, T);
+        hipLaunchKernelGGL(k_attention_merge<64>, dim3(a.heads), dim3(kBlock), 0, s, a, geo.nch);
+    }
+    return a.heads;
+}
+
+// The same in one launch with a workgroup per query head, which needs no
+// partials or counters: the tiled kernels' bits where those apply.
+static void launch_attention_direct(AttnArgs a, const AttnGeo& geo, size_t heads, size_t kvheads, size_t d,
+                                    hipStream_t s) {
+    const bool tiled = attention_shape(a, geo, heads, kvheads, d);
+    const uint32_t T = (uint32_t)geo.T;
+    const dim3 grid(a.heads), any(kAnyBlock);
+    if (tiled && d == 128)
+        hipLaunchKernelGGL(k_attention_direct<128>, grid, dim3(kDirectBlock), 0, s, a, T);
+    else if (tiled)
+        hipLaunchKernelGGL(k_attention_direct<64>, grid, dim3(kDirectBlock), 0, s, a, T);
+    else if (d <= 64)
+        hipLaunchKernelGGL(k_attention_any<8>, grid, any, 0, s, a, T);
+    else if (d <= 128)
+        hipLaunchKernelGGL(k_attention_any<16>, grid, any, 0, s, a, T);
+    else if (d <= 256)
+        hipLaunchKernelGGL(k_attention_any<32>, grid, any, 0, s, a, T);
+    else
+        hipLaunchKernelGGL(k_attention_wide, grid, any, 0, s, a, T);
 }
 
 int qh_attention(qh_ctx* c, const float* q, const float* k, const float* v, size_t klen, size_t heads,
@@ -1783,6 +1856,7 @@ int qh_attention(qh_ctx* c, const float* q, const float* k, const float* v, size
         a.counter = cnt;
         a.out = dout;
         launch_attention(a, geo, heads, kvheads, d, c->s);
+        HIP_OK(hipGetLastError());
         copy_out(c, out, dout, heads * d * 4);
         sync(c);
     });
@@ -1799,16 +1873,35 @@ int qh_attention_noalloc(qh_ctx* c, const float* q, const float* k, const float*
                         " bytes of scratch; the no-allocation entry point holds " +
                         std::to_string(kNoAllocScratchBytes));
         hipStream_t s = stream ? static_cast<hipStream_t>(stream) : c->s;
-        uint8_t* base = noalloc_scratch(c->device, s);
-        uint32_t* cnt = reinterpret_cast<uint32_t*>(base + part_bytes);
         AttnArgs a{};
         a.q = q;
         a.k = k;
         a.v = v;
-        a.part = reinterpret_cast<float*>(base);
-        a.counter = cnt;
         a.out = out;
-        launch_attention(a, geo, heads, kvheads, d, s);
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (stream) HIP_OK(hipStreamIsCapturing(s, &capture));
+        if (capture != hipStreamCaptureStatusNone) {
+            launch_attention_direct(a, geo, heads, kvheads, d, s);
+            HIP_OK(hipGetLastError());
+            return;
+        }
+        {
+            ScratchAreas& S = g_scratch[c->device];
+            std::lock_guard<std::mutex> lock(S.mu);
+            if (!S.base) throw Error("no-allocation scratch is not set up on this device");
+            if (ScratchAreas::Area* A = noalloc_area(S, s)) {
+                const size_t i = A - S.area;
+                uint8_t* base = S.base + i * kNoAllocScratchBytes;
+                a.part = reinterpret_cast<float*>(base);
+                a.counter = reinterpret_cast<uint32_t*>(base + part_bytes);
+                a.done = S.done + i;
+                A->used = ++S.calls;
+                A->launched += launch_attention(a, geo, heads, kvheads, d, s);
+            } else {
+                launch_attention_direct(a, geo, heads, kvheads, d, s);
+            }
+            HIP_OK(hipGetLastError());
+        }
         if (!stream) HIP_OK(hipStreamSynchronize(s));
     });
 }

@@ -251,6 +251,10 @@ __device__ __forceinline__ void attention_block(const AttnArgs& a, uint32_t T) {
         }
         a.out[(g * G + h) * d + j] = O / L;
     }
+    if (a.done) {
+        __syncthreads();
+        if (threadIdx.x == 0) atomicAdd(a.done, 1ull);
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_attention_api(AttnArgs a, uint32_t T) { attention_block(a, T); }
@@ -408,6 +412,7 @@ __global__ __launch_bounds__(kBlock) void k_attention_merge(AttnArgs a, uint32_t
         if (grp + NG * i < nch) O = fmaf(w[grp + NG * i], o[i], O);
     red[grp][j] = O;
     __syncthreads();
+    if (threadIdx.x == 0 && a.done) atomicAdd(a.done, 1ull);  // the partials have been read
     if (grp == 0) {
         for (uint32_t k = 1; k < NG; k++) O += red[k][j];
         a.out[(size_t)blockIdx.x * D + j] = O / L;
@@ -417,5 +422,272 @@ template __global__ void k_attention_tile<64>(AttnArgs, uint32_t);
 template __global__ void k_attention_tile<128>(AttnArgs, uint32_t);
 template __global__ void k_attention_merge<64>(AttnArgs, uint32_t);
 template __global__ void k_attention_merge<128>(AttnArgs, uint32_t);
+
+// k_attention_tile and k_attention_merge in one launch that uses no memory
+// besides its arguments: one workgroup per query head takes the chunks four at
+// a time (four waves each, k_attention_tile's work for one head), keeps their
+// partials in LDS and merges them.  Every sum has the two kernels' terms in
+// their order, so the bits are theirs.
+// Bound by one CU's share of the bandwidth (a head's K and V, 3.7 MB at 3,581
+// keys of 128) and the tiles' barriers: 70 us a graph replay at 32 / 4 heads of
+// 128 and 3,581 keys, 41 at 1,024, 16 at 64 (the two kernels, whose scratch a
+// replay could share with another call: 16, 15, 15).
+template <int D>
+__global__ __launch_bounds__(kDirectBlock) void k_attention_direct(AttnArgs a, uint32_t T) {
+    constexpr int NQ = D / 32, NV = D / 64;
+    constexpr uint32_t kTile = 64, kPW = 16, NC = kDirectBlock / kBlock;  // chunks at a time
+    __shared__ float part[64][D + 2];
+    __shared__ float sc[NC][kTile], ps[NC][kTile], al[NC], red[NC][kWaves][D], w[64];
+    const uint32_t h = blockIdx.x, g = h / (a.heads / a.kvheads), nch = a.max_chunks;
+    const uint32_t cg = threadIdx.x / kBlock, tid = threadIdx.x % kBlock;
+    const uint32_t lane = tid & 63, wv = tid >> 6, kl = lane >> 3, p = lane & 7;
+    const float* kb = a.k + (size_t)g * a.sh;
+    const float* vb = a.v + (size_t)g * a.sh;
+    float4 q[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; i++) q[i] = gld<float4>(a.q + (size_t)h * D + 4 * (p + 8 * i));
+    const float root = sqrtf((float)D);
+    for (uint32_t c0 = 0; c0 < nch; c0 += NC) {  // every thread passes every barrier
+        const uint32_t ch = c0 + cg, k0 = ch * a.span, k1 = min(T, k0 + a.span);
+        const bool live = ch < nch;
+        float acc[NV], m = -INFINITY, l = 0.f;
+#pragma unroll
+        for (int i = 0; i < NV; i++) acc[i] = 0.f;
+        for (uint32_t t = 0; t < a.span; t += kTile) {
+            const uint32_t t0 = k0 + t;
+            const bool on = live && t0 < k1;
+            float4 kr[2][NQ];
+            float vr[kPW][NV];
+            if (on) {
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+#pragma unroll
+                    for (int i = 0; i < NQ; i++)
+                        kr[r][i] =
+                            gld<float4>(kb + (size_t)min(t0 + kPW * wv + 8 * r + kl, k1 - 1) * a.st + 4 * (p + 8 * i));
+#pragma unroll
+                for (uint32_t j = 0; j < kPW; j++) {
+                    const float* row = vb + (size_t)min(t0 + kPW * wv + j, k1 - 1) * a.st;
+                    if constexpr (NV == 2) {
+                        const float2 x = gld<float2>(row + 2 * lane);
+                        vr[j][0] = x.x;
+                        vr[j][1] = x.y;
+                    } else {
+                        vr[j][0] = gld<float>(row + lane);
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    float s = 0.f;
+#pragma unroll
+                    for (int i = 0; i < NQ; i++) {
+                        s = fmaf(q[i].x, kr[r][i].x, s);
+                        s = fmaf(q[i].y, kr[r][i].y, s);
+                        s = fmaf(q[i].z, kr[r][i].z, s);
+                        s = fmaf(q[i].w, kr[r][i].w, s);
+                    }
+#pragma unroll
+                    for (int o = 4; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+                    if (p == 0) sc[cg][kPW * wv + 8 * r + kl] = s;
+                }
+            }
+            __syncthreads();
+            if (on && wv == 0) {
+                const float v = t0 + lane < k1 ? sc[cg][lane] / root : -INFINITY;
+                const float M = fmaxf(m, wave_max(v)), e = expf(v - M), alpha = expf(m - M);
+                l = fmaf(l, alpha, wave_sum(e));
+                m = M;
+                ps[cg][lane] = e;
+                if (lane == 0) al[cg] = alpha;
+            }
+            __syncthreads();
+            if (on) {
+#pragma unroll
+                for (int i = 0; i < NV; i++) acc[i] *= al[cg];
+#pragma unroll
+                for (uint32_t j = 0; j < kPW; j++) {
+                    const float e = ps[cg][kPW * wv + j];
+#pragma unroll
+                    for (int i = 0; i < NV; i++) acc[i] = fmaf(e, vr[j][i], acc[i]);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) red[cg][wv][NV * lane + i] = acc[i];
+        __syncthreads();
+        if (live) {
+            if (tid < D) part[ch][2 + tid] = (red[cg][0][tid] + red[cg][1][tid]) + (red[cg][2][tid] + red[cg][3][tid]);
+            if (tid < 2) part[ch][tid] = tid ? l : m;  // of wave 0
+        }
+    }
+    __syncthreads();
+    constexpr uint32_t NG = kBlock / D, kPer = 64 / NG;
+    float(*rg)[D] = red[0];
+    const uint32_t j = tid % D, grp = tid / D;
+    const bool ok = lane < nch;
+    const uint32_t mine = min(lane, nch - 1);
+    const float mc = ok ? part[mine][0] : -INFINITY, lc = ok ? part[mine][1] : 0.f;
+    const float M = wave_max(mc), e = ok ? expf(mc - M) : 0.f, L = wave_sum(lc * e);
+    if (threadIdx.x < 64) w[lane] = e;
+    __syncthreads();
+    float O = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < kPer; i++)
+        if (grp + NG * i < nch) O = fmaf(w[grp + NG * i], part[grp + NG * i][2 + j], O);
+    if (cg == 0) rg[grp][j] = O;
+    __syncthreads();
+    if (threadIdx.x < D) {
+        for (uint32_t k = 1; k < NG; k++) O += rg[k][j];
+        a.out[(size_t)h * D + j] = O / L;
+    }
+}
+template __global__ void k_attention_direct<64>(AttnArgs, uint32_t);
+template __global__ void k_attention_direct<128>(AttnArgs, uint32_t);
+
+// The same for other shapes of up to 8 E elements a head, without LDS partials:
+// eight lanes share a key, with E elements of its row each, and keep the (m, l,
+// o) of their own keys, so there is no barrier before the merge at the end.
+// Another order of sums than k_attention_api's.
+template <int E>
+__global__ __launch_bounds__(kAnyBlock) void k_attention_any(AttnArgs a, uint32_t T) {
+    constexpr uint32_t kW = kAnyBlock / 64, U = E <= 16 ? 2 : 1;  // waves; keys per lane group and step
+    __shared__ float red[kW][8 * E], rm[kW], rl[kW];
+    const uint32_t h = blockIdx.x, g = h / (a.heads / a.kvheads), d = a.d;
+    const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6, kl = lane >> 3, p = lane & 7;
+    auto load = [&](float (&x)[E], const float* row) {  // elements p + 8 i, 0 past d
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            const float t = gld<float>(row + min(p + 8 * i, d - 1));
+            x[i] = p + 8 * i < d ? t : 0.f;
+        }
+    };
+    float q[E], o[E], m = -INFINITY, l = 0.f;
+    load(q, a.q + (size_t)h * d);
+#pragma unroll
+    for (int i = 0; i < E; i++) o[i] = 0.f;
+    const float root = sqrtf((float)d);
+    for (size_t t0 = 8 * wv; t0 < T; t0 += 8 * kW * U) {  // the wave's first key of the step
+        float kr[U][E], vr[U][E], s[U], M = m;
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) load(kr[u], a.k + g * a.sh + min(t0 + kl + 8 * kW * u, (size_t)T - 1) * a.st);
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) load(vr[u], a.v + g * a.sh + min(t0 + kl + 8 * kW * u, (size_t)T - 1) * a.st);
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            float t = 0.f;
+#pragma unroll
+            for (int i = 0; i < E; i++) t = fmaf(q[i], kr[u][i], t);
+#pragma unroll
+            for (int x = 1; x < 8; x <<= 1) t += __shfl_xor(t, x, 64);
+            s[u] = t0 + kl + 8 * kW * u < T ? t / root : -INFINITY;
+            M = fmaxf(M, s[u]);
+        }
+        const float Mf = M == -INFINITY ? 0.f : M, alpha = expf(m - Mf);  // 0 while no key came
+        m = M;
+        l *= alpha;
+#pragma unroll
+        for (int i = 0; i < E; i++) o[i] *= alpha;
+#pragma unroll
+        for (uint32_t u = 0; u < U; u++) {
+            const float e = expf(s[u] - Mf);
+            if (t0 + kl + 8 * kW * u < T) {  // not 0 times the value of a key past the end
+                l += e;
+#pragma unroll
+                for (int i = 0; i < E; i++) o[i] = fmaf(e, vr[u][i], o[i]);
+            }
+        }
+    }
+    // the wave's eight lane groups, then the waves
+    float M = m;
+#pragma unroll
+    for (int x = 8; x < 64; x <<= 1) M = fmaxf(M, __shfl_xor(M, x, 64));
+    const float e = expf(m - (M == -INFINITY ? 0.f : M));
+    l *= e;
+#pragma unroll
+    for (int i = 0; i < E; i++) o[i] *= e;
+#pragma unroll
+    for (int x = 8; x < 64; x <<= 1) {
+        l += __shfl_xor(l, x, 64);
+#pragma unroll
+        for (int i = 0; i < E; i++) o[i] += __shfl_xor(o[i], x, 64);
+    }
+    if (kl == 0) {
+#pragma unroll
+        for (int i = 0; i < E; i++) red[wv][p + 8 * i] = o[i];
+    }
+    if (lane == 0) {
+        rm[wv] = M;
+        rl[wv] = l;
+    }
+    __syncthreads();
+    if (threadIdx.x < d) {
+        float Ma = -INFINITY, L = 0.f, O = 0.f;
+        for (uint32_t x = 0; x < kW; x++) Ma = fmaxf(Ma, rm[x]);
+        if (Ma == -INFINITY) Ma = 0.f;
+        for (uint32_t x = 0; x < kW; x++) {
+            const float f = expf(rm[x] - Ma);
+            L = fmaf(rl[x], f, L);
+            O = fmaf(red[x][threadIdx.x], f, O);
+        }
+        a.out[(size_t)h * d + threadIdx.x] = O / L;
+    }
+}
+template __global__ void k_attention_any<8>(AttnArgs, uint32_t);
+template __global__ void k_attention_any<16>(AttnArgs, uint32_t);
+template __global__ void k_attention_any<32>(AttnArgs, uint32_t);
+
+// The same for heads of more than 256 elements (the LDS budget of the entry
+// points ends at 4,094): tiles of 64 keys, eight lanes a
+// key for the scores, then a thread per output element and key of the tile.
+__global__ __launch_bounds__(kAnyBlock) void k_attention_wide(AttnArgs a, uint32_t T) {
+    constexpr uint32_t kTile = 64, kMax = 8;  // keys per tile, output elements per thread
+    __shared__ float ps[kTile], al, lsum;
+    const uint32_t h = blockIdx.x, g = h / (a.heads / a.kvheads), d = a.d;
+    const uint32_t lane = threadIdx.x & 63, key = threadIdx.x >> 3, p = threadIdx.x & 7;
+    static_assert(kAnyBlock == 8 * kTile, "eight lanes a key");
+    const float* q = a.q + (size_t)h * d;
+    const float root = sqrtf((float)d);
+    float o[kMax], m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < kMax; i++) o[i] = 0.f;
+    for (size_t t0 = 0; t0 < T; t0 += kTile) {
+        const uint32_t n = (uint32_t)min((size_t)kTile, T - t0);
+        const float* kt = a.k + g * a.sh + (t0 + min(key, n - 1)) * a.st;
+        float s = 0.f;
+        for (uint32_t j = p; j < d; j += 8) s = fmaf(gld<float>(q + j), gld<float>(kt + j), s);
+#pragma unroll
+        for (int x = 1; x < 8; x <<= 1) s += __shfl_xor(s, x, 64);
+        if (p == 0) ps[key] = key < n ? s / root : -INFINITY;
+        __syncthreads();
+        if (threadIdx.x < 64) {
+            const float v = ps[lane], M = fmaxf(m, wave_max(v)), Mf = M == -INFINITY ? 0.f : M;
+            const float e = expf(v - Mf), alpha = expf(m - Mf);
+            l = fmaf(l, alpha, wave_sum(e));
+            m = M;
+            ps[lane] = e;
+            if (lane == 0) {
+                al = alpha;
+                lsum = l;
+            }
+        }
+        __syncthreads();
+        const float* vt = a.v + g * a.sh + t0 * a.st;
+#pragma unroll
+        for (uint32_t i = 0; i < kMax; i++) {
+            const uint32_t j = threadIdx.x + kAnyBlock * i;
+            if (j >= d) break;
+            float x = o[i] * al;
+#pragma unroll 8
+            for (uint32_t t = 0; t < n; t++) x = fmaf(ps[t], gld<float>(vt + t * a.st + j), x);
+            o[i] = x;
+        }
+        __syncthreads();  // the next tile's scores overwrite ps
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kMax; i++) {
+        const uint32_t j = threadIdx.x + kAnyBlock * i;
+        if (j < d) a.out[(size_t)h * d + j] = o[i] / lsum;
+    }
+}
 
 }  // namespace qh

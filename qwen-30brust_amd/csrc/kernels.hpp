@@ -131,7 +131,9 @@ struct AttnArgs {
     uint32_t* counter;  // [kvheads]
     float* out;         // [heads*d]
     uint32_t* err;      // nullable: error bits (kErrContext on a chunk overflow)
+    unsigned long long* done;  // nullable: one more from each workgroup that has merged its partials
 };
+constexpr uint32_t kDirectBlock = 1024, kAnyBlock = 512;  // threads of k_attention_direct, k_attention_any and _wide
 
 // Arguments of the persistent token-step kernel (decode.hip): layers
 // [l0, l1) of one token, followed (vocab = 1) by the vocab projection, argmax
