@@ -1785,7 +1785,8 @@ static bool attention_shape(AttnArgs& a, const AttnGeo& geo, size_t heads, size_
     a.span = geo.span;
     a.err = nullptr;
     const bool aligned = ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v) % 16 == 0;
-    return aligned && (d == 128 || d == 64) && heads / kvheads <= 8;
+    // a tile's 64 rows are addressed with 32-bit byte offsets
+    return aligned && (d == 128 || d == 64) && heads / kvheads <= 8 && kvheads * d * 256 <= 0x7fffffffu;
 }
 
 // Launches the attention of `a` (its q, k, v, part, counter, done and out

@@ -305,15 +305,20 @@ __global__ __launch_bounds__(kBlock) void k_attention_tile(AttnArgs a, uint32_t 
 #pragma unroll
             for (int i = 0; i < NQ; i++)
                 kr[r][i] = gld<float4>(kb + (size_t)min(t0 + kPW * wv + 8 * r + kl, k1 - 1) * a.st + 4 * (p + 8 * i));
+        // values of keys past the end are read as 0, by the bounds of a buffer
+        // resource over the tile: an infinite one times its probability 0 would
+        // be NaN (zeroed behind the loads instead, a call took 0.5 us longer)
+        const __amdgpu_buffer_rsrc_t vt =
+            buf_rsrc(vb + (size_t)t0 * a.st, ((min(k1 - t0, kTile) - 1) * (uint32_t)a.st + D) * 4);
 #pragma unroll
-        for (uint32_t j = 0; j < kPW; j++) {  // keys past the end: the last key again, with probability 0
-            const float* row = vb + (size_t)min(t0 + kPW * wv + j, k1 - 1) * a.st;
+        for (uint32_t j = 0; j < kPW; j++) {
+            const int off = (int)(((kPW * wv + j) * (uint32_t)a.st + NV * lane) * 4);
             if constexpr (NV == 2) {
-                const float2 t = gld<float2>(row + 2 * lane);
+                const float2 t = __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(vt, off, 0, 0));
                 vr[j][0] = t.x;
                 vr[j][1] = t.y;
             } else {
-                vr[j][0] = gld<float>(row + lane);
+                vr[j][0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(vt, off, 0, 0));
             }
         }
 #pragma unroll
@@ -502,6 +507,12 @@ __global__ __launch_bounds__(kDirectBlock) void k_attention_direct(AttnArgs a, u
             }
             __syncthreads();
             if (on) {
+                if (t0 + kPW * wv + kPW > k1) {  // as there: no value past the end
+#pragma unroll
+                    for (uint32_t j = 0; j < kPW; j++)
+#pragma unroll
+                        for (int i = 0; i < NV; i++) vr[j][i] = t0 + kPW * wv + j < k1 ? vr[j][i] : 0.f;
+                }
 #pragma unroll
                 for (int i = 0; i < NV; i++) acc[i] *= al[cg];
 #pragma unroll
