@@ -172,7 +172,8 @@ int qh_forward(qh_ctx *ctx, uint32_t token, float *logits, size_t logits_cap, ui
  * all chained on the device with no per-token host round trip (the
  * src/main.rs:250-282 loop with temperature 0).  out_tokens receives the
  * n_new generated ids; logits_last (room for logits_cap floats, nullable)
- * the logits that produced the last generated token. */
+ * the logits that produced the last generated token.  A call that fails
+ * writes neither. */
 int qh_generate(qh_ctx *ctx, const uint32_t *prompt, size_t n_prompt, size_t n_new,
                 uint32_t *out_tokens, float *logits_last, size_t logits_cap);
 /* == Sampler (src/sampling.rs:3-65) with its rand 0.8.8 StdRng stream
@@ -219,7 +220,7 @@ int qh_position(const qh_ctx *ctx, size_t *out);
  * forwards: the first prompt token at the context limit fails with "context
  * limit N reached", a token outside the vocabulary with "token outside
  * vocabulary" (src/model.rs:219-223), and every failure leaves a clean cache
- * at position 0 (src/model.rs:209-216). */
+ * at position 0 (src/model.rs:209-216) and logits and argmax as they were. */
 int qh_prefill(qh_ctx *ctx, const uint32_t *prompt, size_t n, float *logits, size_t logits_cap,
                uint32_t *argmax);
 /* Prefill implementation (no counterpart in the reference, whose prompt loop

@@ -346,9 +346,12 @@ struct qh_ctx {
     DevBuf sa, sb, sc, sd;
     // transfers of the current call through pinned host memory (copy_in,
     // copy_out): bytes in use, and the caller's buffers to fill after the sync
+    // (from the pinned area, or from device memory where they did not fit)
     struct Out {
         void* dst;
-        size_t off, bytes;
+        const void* src;
+        size_t bytes;
+        bool pinned;
     };
     HostPinned pin;
     size_t pin_used = 0;
@@ -396,7 +399,8 @@ thread_local std::string g_create_err;
 
 template <class F> int guarded(qh_ctx* c, F f) {
     try {
-        if (c && c->pin_used) {  // a call that failed before its sync: its copies end, its outputs are dropped
+        // a call that failed before its sync: its copies end, its outputs are dropped
+        if (c && (c->pin_used || !c->outs.empty())) {
             (void)hipStreamSynchronize(c->s);
             c->pin_used = 0;
             c->outs.clear();
@@ -409,14 +413,28 @@ template <class F> int guarded(qh_ctx* c, F f) {
     }
 }
 
-// Waits for the stream, then hands out what copy_out staged.
-void sync(qh_ctx* c) {
+// sync: waits for the stream (wait), then fills the caller's buffers with what
+// copy_out staged (hand_out).
+void wait(qh_ctx* c) {
     const hipError_t e = hipStreamSynchronize(c->s);
+    c->pin_used = 0;
+    if (e != hipSuccess) c->outs.clear();
+    HIP_OK(e);
+}
+void hand_out(qh_ctx* c) {
     const std::vector<qh_ctx::Out> outs = std::move(c->outs);
     c->outs.clear();
-    c->pin_used = 0;
-    HIP_OK(e);
-    for (const auto& o : outs) std::memcpy(o.dst, static_cast<const uint8_t*>(c->pin.p) + o.off, o.bytes);
+    bool more = false;
+    for (const auto& o : outs) {
+        if (o.pinned) std::memcpy(o.dst, o.src, o.bytes);
+        else HIP_OK(hipMemcpyAsync(o.dst, o.src, o.bytes, hipMemcpyDeviceToHost, c->s));
+        more |= !o.pinned;
+    }
+    if (more) HIP_OK(hipStreamSynchronize(c->s));
+}
+void sync(qh_ctx* c) {
+    wait(c);
+    hand_out(c);
 }
 
 // Device words copied (and dst zero-filled up to `padded`) by a kernel in the
@@ -430,11 +448,12 @@ void launch_stage(qh_ctx* c, void* dst, const void* src, size_t words, size_t pa
 
 // Room for `bytes` in the pinned area until the next sync, or null when this
 // call's transfers do not fit (they then go through hipMemcpyAsync).
-constexpr size_t kPinBytes = 4u << 20;
+// get_state's words lie behind it, so that they always fit.
+constexpr size_t kPinBytes = 4u << 20, kPinState = 256;
 uint8_t* pin_room(qh_ctx* c, size_t bytes) {
     const size_t need = (bytes + 255) / 256 * 256;
     if (c->pin_used + need > kPinBytes) return nullptr;
-    c->pin.reserve(kPinBytes);
+    c->pin.reserve(kPinBytes + kPinState);
     uint8_t* p = static_cast<uint8_t*>(c->pin.p) + c->pin_used;
     c->pin_used += need;
     return p;
@@ -458,10 +477,10 @@ void copy_in(qh_ctx* c, void* dst, const void* src, size_t bytes, size_t padded 
 void copy_out(qh_ctx* c, void* dst, const void* src, size_t bytes) {
     if (uint8_t* p = pin_room(c, bytes)) {
         launch_stage(c, p, src, bytes / 4, bytes / 4);
-        c->outs.push_back({dst, (size_t)(p - static_cast<uint8_t*>(c->pin.p)), bytes});
+        c->outs.push_back({dst, p, bytes, true});
         return;
     }
-    HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->s));
+    c->outs.push_back({dst, src, bytes, false});
 }
 
 // Uploads `rows` packed GGUF rows (src) into device rows at dst, repacking on
@@ -1034,10 +1053,17 @@ void put_state(qh_ctx* c, uint32_t pos, uint32_t n_given, const uint32_t* token 
     HIP_OK(hipGetLastError());
 }
 
-DevState get_state(qh_ctx* c) {
-    DevState st{};
-    copy_out(c, &st, c->acts.st, sizeof st);
-    sync(c);
+// Ends the call's device work: the step state, and the staged outputs to the
+// caller, not after a failed step where `keep` says that it keeps its buffers.
+DevState get_state(qh_ctx* c, bool keep = false) {
+    c->pin.reserve(kPinBytes + kPinState);
+    uint8_t* p = static_cast<uint8_t*>(c->pin.p) + kPinBytes;
+    launch_stage(c, p, c->acts.st, sizeof(DevState) / 4, sizeof(DevState) / 4);
+    wait(c);
+    DevState st;
+    std::memcpy(&st, p, sizeof st);
+    if (st.err && keep) c->outs.clear();
+    hand_out(c);
     return st;
 }
 
@@ -1948,7 +1974,7 @@ int qh_generate(qh_ctx* c, const uint32_t* prompt, size_t n_prompt, size_t n_new
         for (size_t i = 0; i < steps; i++) launch_step(c);
         if (n_new) copy_out(c, out_tokens, c->acts.tokens + c->pos + n_prompt, n_new * 4);
         if (logits_last) copy_out(c, logits_last, c->acts.logits, c->cfg.vocab * 4);
-        DevState st = get_state(c);
+        DevState st = get_state(c, true);
         if (st.err) fail_step(c, st.err);
         c->pos += steps;
         c->stats.matvecs += matvecs_per_token(c) * steps;
@@ -1971,6 +1997,7 @@ int qh_prefill(qh_ctx* c, const uint32_t* prompt, size_t n, float* logits, size_
         try {
             prefill_body(c, prompt, n, logits, logits_cap, argmax, t0);
         } catch (...) {
+            c->outs.clear();
             try {
                 reset_model(c);
             } catch (...) {
@@ -1996,7 +2023,7 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
             put_state(c, (uint32_t)c->pos, (uint32_t)(c->pos + n));
             for (size_t i = 0; i < n; i++) launch_step(c);
             if (logits) copy_out(c, logits, c->acts.logits, c->cfg.vocab * 4);
-            DevState st = get_state(c);
+            DevState st = get_state(c, true);
             if (st.err) fail_step(c, st.err);
             if (argmax) *argmax = st.argmax;
             c->pos += n;
@@ -2035,7 +2062,7 @@ static void prefill_body(qh_ctx* c, const uint32_t* prompt, size_t n, float* log
         enqueue_tail(c);
         HIP_OK(hipGetLastError());
         if (logits) copy_out(c, logits, c->acts.logits, c->cfg.vocab * 4);
-        DevState st = get_state(c);
+        DevState st = get_state(c, true);
         if (st.err) {
             // the prompt's tokens and positions were checked above, so this is
             // numeric: an fp16 operand out of range (kErrRange), or router
