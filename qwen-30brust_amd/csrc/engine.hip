@@ -462,6 +462,7 @@ uint8_t* pin_room(qh_ctx* c, size_t bytes) {
 // Caller memory to the device, dst zero-filled up to `padded` bytes; whole
 // 32-bit words are written.
 void copy_in(qh_ctx* c, void* dst, const void* src, size_t bytes, size_t padded = 0) {
+    if (bytes && !src) throw Error("null input buffer");
     padded = std::max((bytes + 3) / 4 * 4, padded);
     if (padded == 0) return;
     if (uint8_t* p = pin_room(c, bytes)) {
@@ -475,6 +476,8 @@ void copy_in(qh_ctx* c, void* dst, const void* src, size_t bytes, size_t padded 
 
 // Device memory (whole words) to the caller's, there after the next sync(c).
 void copy_out(qh_ctx* c, void* dst, const void* src, size_t bytes) {
+    if (bytes == 0) return;
+    if (!dst) throw Error("null output buffer");
     if (uint8_t* p = pin_room(c, bytes)) {
         launch_stage(c, p, src, bytes / 4, bytes / 4);
         c->outs.push_back({dst, p, bytes, true});
@@ -1740,6 +1743,7 @@ int qh_route(qh_ctx* c, const float* logits, size_t n, size_t top, uint32_t* ids
         copy_out(c, h.data(), dids, h.size() * 4);
         sync(c);
         if (h.back()) throw Error("invalid MoE router");
+        if (!ids || !w) throw Error("null output buffer");
         std::memcpy(ids, h.data(), top * 4);
         std::memcpy(w, h.data() + pad32h(top), top * 4);
     });
