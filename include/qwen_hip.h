@@ -214,7 +214,8 @@ int qh_position(const qh_ctx *ctx, size_t *out);
  * operands with fp32 accumulation (logits within about 1e-2 relative of the
  * FP32 path).  Models the batched path does not cover (head_dim != 128, more
  * than 8 query heads per KV head, more than 128 experts, widths that are not
- * whole 256-column super-blocks, projections that are not block-quantised)
+ * whole 256-column super-blocks (a query width of whole pairs of them),
+ * projections that are not block-quantised)
  * run the prompt through the exact token step instead, one per token on the
  * device (the same bits as n qh_forward calls).  Errors as that loop of
  * forwards: the first prompt token at the context limit fails with "context

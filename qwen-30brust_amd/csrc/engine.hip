@@ -1110,8 +1110,9 @@ std::string prefill_gap(const qh_ctx* c) {
     if (d.heads % d.kvheads || d.heads / d.kvheads > 8) return "more than 8 query heads per KV head";
     if (d.experts > 128) return "more than 128 experts";
     if (d.hidden % 256 || d.ff % 256) return "hidden or expert width not a multiple of 256";
-    // the o-projection runs as two column halves, each whole 256-column
-    // super-blocks (and an even number of 64-column GEMM slices)
+    // pf_dense itself needs whole 256-column super-blocks only; an odd number
+    // of them stays with the exact step, as when the o-projection always ran as
+    // two column halves (the batched path is checked for even numbers)
     if ((d.heads * 128) % 512) return "query width not a multiple of 512";
     for (const LayerW& L : c->layers) {
         if (!(km(L.q.kind) && km(L.k.kind) && km(L.v.kind) && km(L.o.kind) && km(L.gate.kind) &&

@@ -244,9 +244,10 @@ def test_prefill_uncovered_model_runs_the_exact_step(dev):
 
 
 def test_prefill_odd_query_width_runs_the_exact_step(dev):
-    """Two query heads (query width 256): the o-projection's two column halves
-    would not be whole super-blocks, so the batched path leaves the model to
-    the exact token step (bit-equal to a stepwise forward) instead of failing."""
+    """Two query heads (query width 256, an odd number of 256-column
+    super-blocks, which two equal column splits would not leave whole): the
+    batched path leaves the model to the exact token step (bit-equal to a
+    stepwise forward) instead of failing."""
     spec = synth.Spec(256, 1, 2, 1, 128, 8, 2, 256, 256, 64, types=synth._k_types(), seed=5)
     img = synth.build_image(spec)
     prompt = np.random.default_rng(3).integers(0, spec.vocab, 9).astype(np.uint32)
