@@ -169,12 +169,15 @@ constexpr uint32_t kSeg = 16;
 constexpr int kSat = 1 << 26;  // saturation of a map's sums: past 2^24 only "left the binade" matters
 enum : uint32_t { kEvNone = 0u, kEvCross = 1u, kEvHit = 2u, kEvStall = 3u };
 
+constexpr uint32_t kSerialCut = 640, kSerialAll = 256;  // most ids folded by one lane (pick_rank)
+
 struct FoldLds {
     int w0[kSW], w1[kSW];
     uint32_t first;   // first thread with an event
     uint32_t kind;    // its event
     uint32_t at;      // element index of a hit
     float s;          // the fold's value after that thread
+    float head[kSerialCut];  // the probabilities of a serial fold
 };
 
 // A then B.
@@ -305,20 +308,25 @@ __device__ __forceinline__ float fold(FoldLds& F, uint32_t K, float s, X x, Hit 
 // sampling.rs:47-62 over the K sorted probabilities p(i): total, the top-p
 // cut m, the kept mass (a prefix of the total's fold: its value before segment
 // i is kept in seg[i]), the walk.  Returns the picked rank in every thread.
-// A few ids (kSerial: three rounds of fold() cost more than their serial
-// steps) are folded by one lane.
-constexpr uint32_t kSerial = 128;
+// A few ids are folded by one lane: up to kSerialCut where a top-p cut ends its
+// second loop early, up to kSerialAll without one.  It takes 0.05-0.1 us an id,
+// a fold() about 10 us and more over flat probabilities.  A draw from 2,000
+// (32,000) host logits, one lane / three folds: top_p 0.95, top_k 256 52 / 64
+// (71 / 84) us, 512 73 / 77 (95 / 97), 700 81 / 82 (111 / 101); top_p 1, 256
+// 60 / 65 (75 / 85), with a few likely ids 59 / 57 (62 / 60), 384 72 / 59 (83 / 70).
 template <class P>
 __device__ __forceinline__ uint32_t pick_rank(FoldLds& F, uint32_t K, const SampleArgs& a, P p, float* seg,
                                               uint32_t& m_out) {
 #pragma clang fp contract(off)
-    if (K <= kSerial) {
+    if (K <= (a.top_p < 1.f ? kSerialCut : kSerialAll)) {
+        for (uint32_t i = threadIdx.x; i < K; i += kST) F.head[i] = p(i);
+        __syncthreads();
         if (threadIdx.x == 0) {
             float total = -0.0f, cumulative = 0.f, kept = -0.0f;
-            for (uint32_t i = 0; i < K; i++) total += p(i);
+            for (uint32_t i = 0; i < K; i++) total += F.head[i];
             uint32_t m = K, r = 0;
             for (uint32_t i = 0; i < K; i++) {
-                const float x = p(i);
+                const float x = F.head[i];
                 cumulative += x / total;
                 kept += x;
                 if (cumulative >= a.top_p) {
@@ -328,7 +336,7 @@ __device__ __forceinline__ uint32_t pick_rank(FoldLds& F, uint32_t K, const Samp
             }
             float draw = a.draw * kept;
             for (; r < m; r++) {
-                const float x = p(r);
+                const float x = F.head[r];
                 if (draw < x) break;
                 draw -= x;
             }

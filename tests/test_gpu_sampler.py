@@ -141,3 +141,15 @@ def test_sampler_folds(dev, shape, n, t, k, p):
     inside and at the ends of segments: the oracle's ids exactly."""
     got, want = run_both(dev, shape(n), seed=n + k, t=t, k=k, p=p, steps=8)
     assert got == want
+
+
+@pytest.mark.parametrize("shape", [_flat, _levels, _ramp, _peak])
+@pytest.mark.parametrize("n,k,p", [(2000, 256, 1.0), (256, 0, 1.0), (2000, 257, 1.0), (257, 0, 1.0), (2000, 640, 0.3),
+                                   (640, 0, 0.99), (2000, 641, 0.99), (641, 0, 0.3), (9000, 640, 0.9),
+                                   (9000, 641, 0.9), (9000, 256, 1.0)])
+def test_sampler_serial_folds(dev, shape, n, k, p):
+    """Around the most ids that one lane folds, with a top-p cut (640) and
+    without (256), sorted in LDS or (9,000 equal keys) in HBM: the oracle's ids
+    exactly."""
+    got, want = run_both(dev, shape(n), seed=n + k, t=1.0, k=k, p=p, steps=8)
+    assert got == want
