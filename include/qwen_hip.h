@@ -156,7 +156,7 @@ int qh_attention(qh_ctx *ctx, const float *q, const float *k, const float *v, si
  * runs without scratch, with the same bits for head_dim 64 or 128, at most
  * eight query heads per KV head and q, k and v aligned to 16 bytes, else with
  * its sums in another order.  It is slower then for long histories (3,581
- * keys, 32 / 4 heads of 128: 70 us, 8 with an area).  A stream is destroyed
+ * keys, 32 / 4 heads of 128: 70 us, 11 with an area).  A stream is destroyed
  * only when its calls have ended. */
 int qh_attention_noalloc(qh_ctx *ctx, const float *q, const float *k, const float *v, size_t klen,
                          size_t heads, size_t kvheads, size_t d, float *out, void *stream);

@@ -269,8 +269,9 @@ __global__ __launch_bounds__(kBlock) void k_attention_api(AttnArgs a, uint32_t T
 // one wave over the tile's keys; each wave adds its own 16 keys to all heads'
 // outputs.  The chunks are merged by a second launch with a workgroup per head
 // (k_attention_merge): merged by the last workgroup of each KV head, four
-// workgroups read all the partials.  32 / 4 heads of 128, 3,581 keys, both
-// launches: 71-119 -> 8 us a call back to back (tile 8.2, merge 3.9 us alone).
+// workgroups read all the partials.  32 / 4 heads of 128, 3,581 keys:
+// k_attention_api 158 us a call on one stream, these two 11 (tile 8.1, merge
+// 3.8 alone), and 7-8 in turn on three streams, which overlap.
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_attention_tile(AttnArgs a, uint32_t T) {
     constexpr int NQ = D / 32, NV = D / 64;  // float4s of a key's row per lane, dims per lane of a V row
@@ -436,7 +437,7 @@ template __global__ void k_attention_merge<128>(AttnArgs, uint32_t);
 // Bound by one CU's share of the bandwidth (a head's K and V, 3.7 MB at 3,581
 // keys of 128) and the tiles' barriers: 70 us a graph replay at 32 / 4 heads of
 // 128 and 3,581 keys, 41 at 1,024, 16 at 64 (the two kernels, whose scratch a
-// replay could share with another call: 16, 15, 15).
+// replay could share with another call: 16, 15, 15; of an eager call each 10-11).
 template <int D>
 __global__ __launch_bounds__(kDirectBlock) void k_attention_direct(AttnArgs a, uint32_t T) {
     constexpr int NQ = D / 32, NV = D / 64;

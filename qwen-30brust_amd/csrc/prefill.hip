@@ -705,8 +705,8 @@ __global__ __launch_bounds__(kGT, 2) void k_gemm_down(const _Float16* Hs, Expert
 // k_gemm_gateup and k_gemm_down on tiles of 32 MB rows (the work list of a
 // prompt whose experts get few tokens each).  Bound by the experts' weight
 // bytes (226 MB of gate and up rows per layer when every expert is used): at
-// 24 tokens (about 100 experts, 179 MB) gate/up take 41 us per layer, down 21-27
-// us, against 53 and 32-37 us on 128-row tiles.
+// 24 tokens (about 100 experts, 179 MB) gate/up take 47-50 us per layer, down 24-29
+// us, against 61-69 and 31-35 us on 128-row tiles.
 template <uint32_t KIND, int MB>
 __global__ __launch_bounds__(kGT, 3 - (MB - 1)) void k_gemm_gateup_skinny(const _Float16* Xn, uint32_t H, ExpertTiles G,
                                                                           DevMat Wg, DevMat Wu, _Float16* Hs,
@@ -845,7 +845,7 @@ __global__ __launch_bounds__(kGT, 3) void k_gemm_dense(const _Float16* X16, uint
 
 // k_gemm_dense for S <= 32 MB tokens (one row tile): gridDim.x column tiles x
 // gridDim.z column splits of whole super-blocks.  Bound by one round trip for
-// the weights (4.7-5.9 MB per launch): at 24 tokens a launch takes 5.4-6.4 us,
+// the weights (4.7-5.9 MB per launch): at 24 tokens a launch takes 6.1-6.7 us,
 // against 26-33 us in k_gemm_dense with 40 workgroups on one XCD.
 template <uint32_t KIND, int MB>
 __device__ __forceinline__ void dense_skinny_body(const _Float16* X16, uint32_t S, const DevMat& W, uint32_t n0,

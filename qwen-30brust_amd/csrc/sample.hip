@@ -22,8 +22,8 @@
 //
 // Bound: latency.  The data is 608 KB of logits (plus 152 KB of mask); one
 // workgroup walking it alone took about 20 us a pass, five passes a draw.
-// A draw from 151,936 host logits, their upload (about 50 us) included: top_k
-// 20 372 -> 72 us, the whole support 2.3-3.3 ms -> 0.22-0.25 ms.
+// A draw from 151,936 host logits, their copy to the device (22 us of kernels)
+// included: top_k 20 372 -> 61 us, the whole support 2.3-3.3 ms -> 0.20-0.25 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
