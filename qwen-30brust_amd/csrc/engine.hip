@@ -192,7 +192,7 @@ uint64_t groups_host(uint64_t rows, uint64_t cols, int R) {
 // partials counts in `scratch_done`, and the host compares the count with the
 // calls' total.  It does so only for such a stream, because an event behind
 // every call, the other way to know, costs more: 8.1 -> 10.4 us a call over
-// 3,581 keys in turn on three streams (a stream without an area: 21).  A call waits for no other call: where every
+// 3,581 keys in turn on three streams (on 9 to 32 streams: 12).  A call waits for no other call: where every
 // area is in use, and under graph capture (a graph may be launched any number
 // of times, on any stream, beside any call), the attention runs without
 // scratch (launch_attention_direct).  Area and kernels are taken under the
@@ -246,13 +246,32 @@ static void noalloc_init(int device) {
     };
     S.done = static_cast<unsigned long long*>(address(HIP_SYMBOL(scratch_done)));
     if (!S.seen) HIP_OK(hipHostMalloc((void**)&S.seen, sizeof(scratch_done)));
+    std::memset(S.seen, 0, sizeof(scratch_done));
     if (!S.probe) HIP_OK(hipStreamCreateWithFlags(&S.probe, hipStreamNonBlocking));
     S.base = static_cast<uint8_t*>(address(HIP_SYMBOL(scratch)));
 }
 
+// Copies S.done to S.seen; false where that takes over 0.2 ms (about 12 us
+// otherwise): the copy may share a hardware queue with a stream that waits for
+// something this thread has yet to do.  Another thread's capture does not mind
+// the calls (relaxed mode).
+static bool noalloc_probe(ScratchAreas& S) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    hipError_t e = hipStreamQuery(S.probe);  // an earlier copy
+    if (e == hipSuccess) e = hipMemcpyAsync(S.seen, S.done, kNoAllocAreas * 8, hipMemcpyDeviceToHost, S.probe);
+    if (e == hipSuccess) {
+        const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+        while ((e = hipStreamQuery(S.probe)) == hipErrorNotReady && std::chrono::steady_clock::now() < end) {
+        }
+    }
+    (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return e == hipSuccess;
+}
+
 // The area for a call on stream s, or null where other streams' calls use all
-// of them (or where that cannot be found out: another thread's capture may
-// forbid the copy).  The caller holds the lock.
+// of them (or where that cannot be found out).  The caller holds the lock.
 static ScratchAreas::Area* noalloc_area(ScratchAreas& S, hipStream_t s) {
     const uint64_t thread = s == hipStreamPerThread ? thread_serial() : 0;
     ScratchAreas::Area* mine = nullptr;
@@ -260,12 +279,9 @@ static ScratchAreas::Area* noalloc_area(ScratchAreas& S, hipStream_t s) {
         if (A.used && A.stream == s && A.thread == thread) return &A;
         if (!A.used && !mine) mine = &A;
     }
-    if (!mine) {
-        if (hipMemcpyAsync(S.seen, S.done, sizeof(scratch_done), hipMemcpyDeviceToHost, S.probe) != hipSuccess ||
-            hipStreamSynchronize(S.probe) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
+    // first by the last copy: what had ended then and was not called since
+    for (int probes = 0; !mine && probes < 2; probes++) {
+        if (probes == 1 && !noalloc_probe(S)) break;
         for (int i = 0; i < kNoAllocAreas; i++)
             if (S.seen[i] == S.area[i].launched && (!mine || S.area[i].used < mine->used)) mine = &S.area[i];
     }
