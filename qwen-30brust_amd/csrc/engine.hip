@@ -192,14 +192,14 @@ uint64_t groups_host(uint64_t rows, uint64_t cols, int R) {
 // partials counts in `scratch_done`, and the host compares the count with the
 // calls' total.  It does so only for such a stream, because an event behind
 // every call, the other way to know, costs more: 8.1 -> 10.4 us a call over
-// 3,581 keys in turn on three streams (on 9 to 32 streams: 12).  A call waits for no other call: where every
-// area is in use, and under graph capture (a graph may be launched any number
-// of times, on any stream, beside any call), the attention runs without
-// scratch (launch_attention_direct).  Area and kernels are taken under the
-// lock: two host threads that use one stream must not interleave their
-// kernels.  Host code uses only the per-device addresses that
-// hipGetSymbolAddress returns (the arrays' names are host-side stand-ins, not
-// device addresses).
+// 3,581 keys in turn on three streams (on 9 to 32 streams: 12).  A call waits
+// for no other call: where every area is in use, and under graph capture (a
+// graph may be launched any number of times, on any stream, beside any call),
+// the attention runs without scratch (launch_attention_direct).  Area and
+// kernels are taken under the lock: two host threads that use one stream must
+// not interleave their kernels.  Host code uses only the per-device addresses
+// that hipGetSymbolAddress returns (the arrays' names are host-side stand-ins,
+// not device addresses).
 namespace {
 constexpr size_t kNoAllocScratchBytes = 1u << 20;
 constexpr int kNoAllocAreas = 8;

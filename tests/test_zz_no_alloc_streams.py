@@ -69,7 +69,7 @@ def capture(dev, q, k, v, out, klen, shape, stream, execs):
 
 @pytest.mark.parametrize("keys,heads,kvheads,d,off", [
     (1, 4, 4, 128, 0), (65, 32, 4, 128, 0), (4097, 14, 2, 64, 0), (7001, 10, 2, 128, 0), (257, 18, 2, 128, 0), (700, 32, 4, 128, 1),
-    (129, 6, 3, 64, 1), (300, 4, 2, 96, 0), (33, 5, 1, 32, 0), (513, 4, 2, 256, 0), (90, 3, 1, 320, 0), (7, 2, 2, 1, 0)])
+    (129, 6, 3, 64, 1), (300, 4, 2, 96, 0), (33, 5, 1, 32, 0), (513, 4, 2, 256, 0), (90, 3, 1, 320, 0), (70, 1, 1, 4094, 0), (7, 2, 2, 1, 0)])
 def test_captured_call(dev, keys, heads, kvheads, d, off):
     """A captured call's replays against float64, as test_attention_shapes, and
     with the eager call's bits where the register-tiled kernels apply; `off`
